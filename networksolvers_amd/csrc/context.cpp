@@ -342,7 +342,10 @@ int nsmi_ctx_destroy(nsmi_ctx* ctx) {
   // call on this context starts after this one
   std::lock_guard<std::recursive_mutex> lock(ctx->mu);
   (void)hipSetDevice(ctx->device);
-  if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+  if (ctx->stream) {
+    (void)hipStreamSynchronize(ctx->stream);
+    nsmi::xcd_places_release(ctx->device, ctx->stream);
+  }
   for (auto& r : ctx->recs) {
     (void)hipEventDestroy(r.a);
     (void)hipEventDestroy(r.b);
@@ -351,6 +354,7 @@ int nsmi_ctx_destroy(nsmi_ctx* ctx) {
   nsmi::tuner_free(ctx);
   for (size_t j = 0; j < ctx->aux_stream.size(); ++j) {
     (void)hipStreamSynchronize(ctx->aux_stream[j]);
+    nsmi::xcd_places_release(ctx->device, ctx->aux_stream[j]);
     if (j < ctx->aux_blas.size()) rocblas_destroy_handle(ctx->aux_blas[j]);
     if (j < ctx->aux_info.size()) (void)hipFree(ctx->aux_info[j]);
     (void)hipStreamDestroy(ctx->aux_stream[j]);

@@ -7,6 +7,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <functional>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -434,6 +435,13 @@ bool sytrd_launch(nsmi_ctx* ctx, double* A, int n, double* d, double* e, double*
 // zeroes a reduction's barrier and flag words (256 bytes); raises the timeout flag
 // (word 32) when the context has an injected timeout pending and the grid has G > 1
 void reduction_flags_reset(nsmi_ctx* ctx, unsigned* flags, int G);
+// runs launch(xcd) for a kernel whose group of at most 32 workgroups (two of them to a CU)
+// runs on one XCD: the stream's place among the XCDs, see bidiag.hip
+void launch_on_one_xcd(nsmi_ctx* ctx, const std::function<void(int)>& launch);
+void xcd_places_release(int device, hipStream_t stream);
+// start value of a reduction's failure flag: 1 when the context has an injected timeout
+// pending and the grid has G > 1
+unsigned reduction_fail0(nsmi_ctx* ctx, int G);
 void sytrd_check(const SytrdRun& run);
 // Zr <- (Q Z) with Q = H_0 ... H_{n-2} the reflectors of sytrd_launch's output (rho,
 // tau; n <= 1024) and Z = Zr^T (Zr: k x n row-major, i.e. Z column-major n x k): what

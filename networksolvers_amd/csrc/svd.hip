@@ -1,11 +1,8 @@
 // The truncation's own dense eigensolver and SVD (inserter.jl:23 -> ITensors
 // factorize -> LAPACK gesdd on the "svd" route, syevd on the "eigen" route):
 //
-//  * k_bidiag: Householder bidiagonalisation X = Q_L B Q_R^T of a tall r x s
-//    matrix (r >= s, s <= 2048, r <= 4096, r <= 2048 for s > 1024) in one launch,
-//    one grid barrier per column (two where the grid passes 64 workgroups)
-//    (LAPACK dgebrd semantics: upper bidiagonal B, left reflector
-//    H_j on X(j:r, j), right reflector G_j on X(j, j+1:s));
+//  * k_bidiag (bidiag.h): Householder bidiagonalisation X = Q_L B Q_R^T of a tall r x s
+//    matrix (r >= s, s <= 2048, r <= 4096, r <= 2048 for s > 1024) in one launch;
 //  * k_tri_bisect: eigenvalues of a symmetric tridiagonal matrix by Sturm-count
 //    multisection, one wave per eigenvalue.  Applied to the Golub-Kahan matrix of
 //    B (zero diagonal, off-diagonal d_0, e_0, d_1, e_1, ...; eigenvalues +-sigma)
@@ -29,323 +26,6 @@ namespace {
 
 constexpr double kEps = 2.220446049250313e-16;
 constexpr double kSafeMin = 2.2250738585072014e-308;
-
-// ---------------------------------------------------------------- bidiagonalisation
-//
-// Distribution: workgroup g owns the rows i = (4 s + w) G + g of X, slot s of
-// wave w, in registers; lane l holds the columns l + 64 q.  Step j:
-//   A. every row owner takes its x_i = X(i, j) (i > j); each workgroup forms the
-//      partial sums S_c = sum_{own i > j} x_i X(i, c) (c > j) and sigma^2 =
-//      sum x_i^2, and the owner of row j publishes that row (before the update);
-//   grid barrier;
-//   B. every workgroup adds the G partial sums and forms the left reflector
-//      (alpha = X(j, j), beta = -sign(alpha) sqrt(alpha^2 + sigma^2), tau_L =
-//      (beta - alpha) / beta, u = [1, x / (alpha - beta)]), z = u^T X(j:, j+1:) =
-//      X(j, c) + S_c / (alpha - beta), and updates its rows: X(i, c) -= tau_L u_i z_c;
-//      row j after the update, y_c = X(j, c) - tau_L z_c, gives the right reflector
-//      (formed redundantly by every wave), which each owner applies to its rows:
-//      X(i, c) -= tau_R (X(i, :) . v) v_c.
-// Output in place: X(i, j) = u_j[i] for i > j, X(j, j) = d_j, X(j, j+1) = e_j,
-// X(j, c) = v_j[c] for c > j + 1; d, e, tau_L, tau_R.  The exchange buffers (row j,
-// sigma^2 partials, S partials) alternate by the parity of j, as in the tridiagonal
-// reduction.  SINGLE: one workgroup, exchange in LDS, workgroup barriers.
-// TWO (grids of 65 to 256 workgroups): every workgroup reading all G partial
-// rows would move G^2 s doubles per column, so the exchange goes in two levels: after
-// the first barrier workgroup g adds the G partials of its own slice of columns (the
-// reduced vector RS, each column summed once, in a fixed order), and after a second
-// barrier every workgroup reads the reduced vector.
-template <int CL, int RW, bool SINGLE, bool TWO = false>
-__global__ __launch_bounds__(256) void k_bidiag(double* __restrict__ X, int r, int s, double* __restrict__ d,
-                                                double* __restrict__ e, double* __restrict__ tauL,
-                                                double* __restrict__ tauR, double* __restrict__ xch, unsigned* bar,
-                                                unsigned* fail) {
-  constexpr int NP = 64 * CL;
-  __shared__ double comb[4][NP];
-  __shared__ double ys[NP], zs[NP];
-  __shared__ double sgw[4];
-  __shared__ double s_sig;
-  __shared__ int s_ok;
-  const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  double* const Yx = xch;          // [2][s]
-  double* const SG = xch + 2 * s;  // [2][G]
-  double* const PS = SG + 2 * G;   // [2][G][s]
-  double* const RS = PS + 2 * size_t(G) * s;  // [2][s] (TWO)
-
-  double row[RW][CL];
-  int rid[RW];
-#pragma unroll
-  for (int sl = 0; sl < RW; ++sl) {
-    const int i = (sl * 4 + wave) * G + g;
-    rid[sl] = i < r ? i : -1;
-#pragma unroll
-    for (int q = 0; q < CL; ++q) {
-      const int c = lane + 64 * q;
-      row[sl][q] = (i < r && c < s) ? X[size_t(i) * s + c] : 0.0;
-    }
-  }
-  bool finite = true;
-  unsigned nbar = 0;
-  for (int j = 0; j < s; ++j) {
-    const int p = j & 1;
-    const int jq = j >> 6, jl = j & 63;
-    if (SINGLE) __syncthreads();  // the previous step's reads of ys / zs are done
-    // A. column j of the own rows (uniform per wave), partial sums
-    double xi[RW];
-    double sgp = 0.0;
-#pragma unroll
-    for (int sl = 0; sl < RW; ++sl) {
-      double v = 0.0;
-#pragma unroll
-      for (int q = 0; q < CL; ++q)
-        if (q == jq) v = row[sl][q];
-      v = lane_bcast(v, jl);
-      xi[sl] = rid[sl] > j ? v : 0.0;
-      sgp += xi[sl] * xi[sl];
-    }
-#pragma unroll
-    for (int q = 0; q < CL; ++q) {
-      double acc = 0.0;
-#pragma unroll
-      for (int sl = 0; sl < RW; ++sl) acc += xi[sl] * row[sl][q];
-      comb[wave][lane + 64 * q] = acc;
-    }
-    if (lane == 0) sgw[wave] = sgp;
-#pragma unroll
-    for (int sl = 0; sl < RW; ++sl) {
-      if (rid[sl] != j) continue;  // uniform per wave
-#pragma unroll
-      for (int q = 0; q < CL; ++q) {
-        const int c = lane + 64 * q;
-        if (c >= j && c < s) {
-          if (SINGLE)
-            ys[c] = row[sl][q];
-          else
-            Yx[p * s + c] = row[sl][q];
-        }
-      }
-    }
-    __syncthreads();
-    if (SINGLE) {
-      for (int c = tid; c < s; c += 256) zs[c] = (comb[0][c] + comb[1][c]) + (comb[2][c] + comb[3][c]);
-      if (tid == 0) s_sig = (sgw[0] + sgw[1]) + (sgw[2] + sgw[3]);
-      __syncthreads();
-    } else {
-      for (int c = tid; c < s; c += 256)
-        if (c > j) PS[(size_t(p) * G + g) * s + c] = (comb[0][c] + comb[1][c]) + (comb[2][c] + comb[3][c]);
-      if (tid == 0) SG[p * G + g] = (sgw[0] + sgw[1]) + (sgw[2] + sgw[3]);
-      if (!grid_barrier(bar, unsigned(G), ++nbar, fail, &s_ok)) return;
-      if (TWO) {
-        // this workgroup's slice [c0, c1) of the reduced vector: thread t adds the
-        // partials g' = t / 8 + 32 i (G <= 256) of column c0 + t % 8 + 8 b, all loads in
-        // flight; the 32 sums of a column are added in a fixed order
-        const int chunk = (s + G - 1) / G, c0 = g * chunk, c1 = min(s, c0 + chunk);
-        for (int cb = c0; cb < c1; cb += 8) {
-          const int c = cb + (tid & 7);
-          const bool live = c < c1 && c > j;
-          double v[8];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const int gg = (tid >> 3) + 32 * i;
-            v[i] = (live && gg < G) ? PS[(size_t(p) * G + gg) * s + c] : 0.0;
-          }
-          double acc = 0.0;
-#pragma unroll
-          for (int i = 0; i < 8; ++i) acc += v[i];
-          double* const cf = &comb[0][0];  // 256 of the 4 * NP >= 256 entries
-          cf[tid] = acc;
-          __syncthreads();
-          if (tid < 8 && live) {
-            double t = 0.0;
-            for (int k = 0; k < 32; ++k) t += cf[8 * k + tid];
-            RS[size_t(p) * s + c] = t;
-          }
-          __syncthreads();
-        }
-        // sigma^2: the G partials, one wave sum (every workgroup forms the same bits)
-        double sv = 0.0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) sv += lane + 64 * i < G ? SG[p * G + lane + 64 * i] : 0.0;
-        const double sg_all = wave_total(sv);
-        if (!grid_barrier(bar, unsigned(G), ++nbar, fail, &s_ok)) return;
-        constexpr int NY = (NP + 255) / 256;
-        double yv[NY], zv[NY];
-#pragma unroll
-        for (int u = 0; u < NY; ++u) {
-          const int c = tid + 256 * u;
-          yv[u] = (c >= j && c < s) ? Yx[p * s + c] : 0.0;
-          zv[u] = (c > j && c < s) ? RS[size_t(p) * s + c] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < NY; ++u) {
-          const int c = tid + 256 * u;
-          if (c >= j && c < s) ys[c] = yv[u];
-          if (c > j && c < s) zs[c] = zv[u];
-        }
-        if (tid == 0) s_sig = sg_all;
-        __syncthreads();
-      } else {
-      // Every load of the exchange is issued before any is used (one memory round trip
-      // after the barrier): row j (ys), the sigma^2 partials (one per lane), and the G
-      // partial sums of every column, wave w taking the workgroups g = w, w + 4, ...,
-      // NB of them per round (NB * CL loads in flight per lane), added in a fixed
-      // order; the four waves' sums are added in a fixed order below.  Every workgroup
-      // forms the same bits.
-      constexpr int NY = (NP + 255) / 256, NB = CL >= 32 ? 1 : 32 / CL;
-      double yv[NY];
-#pragma unroll
-      for (int u = 0; u < NY; ++u) {
-        const int c = tid + 256 * u;
-        yv[u] = (c >= j && c < s) ? Yx[p * s + c] : 0.0;
-      }
-      const double sgv = lane < G ? SG[p * G + lane] : 0.0;
-      {
-        double acc[CL];
-#pragma unroll
-        for (int q = 0; q < CL; ++q) acc[q] = 0.0;
-        const double* src = PS + size_t(p) * G * s;
-        for (int g0 = wave; g0 < G; g0 += 4 * NB) {
-          double v[NB][CL];
-#pragma unroll
-          for (int bb = 0; bb < NB; ++bb) {
-            const int gg = g0 + 4 * bb;
-#pragma unroll
-            for (int q = 0; q < CL; ++q) {
-              const int c = lane + 64 * q;
-              v[bb][q] = (gg < G && c > j && c < s) ? src[size_t(gg) * s + c] : 0.0;
-            }
-          }
-#pragma unroll
-          for (int bb = 0; bb < NB; ++bb)
-#pragma unroll
-            for (int q = 0; q < CL; ++q) acc[q] += v[bb][q];
-        }
-#pragma unroll
-        for (int q = 0; q < CL; ++q) comb[wave][lane + 64 * q] = acc[q];
-      }
-#pragma unroll
-      for (int u = 0; u < NY; ++u) {
-        const int c = tid + 256 * u;
-        if (c >= j && c < s) ys[c] = yv[u];
-      }
-      const double sg_all = wave_total(sgv);
-      __syncthreads();
-      for (int c = tid; c < s; c += 256)
-        if (c > j) zs[c] = (comb[0][c] + comb[1][c]) + (comb[2][c] + comb[3][c]);
-      if (tid == 0) s_sig = sg_all;
-      __syncthreads();
-      }
-    }
-    // B. left reflector and update
-    const double alpha = ys[j], sig2 = s_sig;
-    double tl = 0.0, beta = alpha, scal = 0.0;
-    if (sig2 != 0.0) {
-      beta = -copysign(sqrt(alpha * alpha + sig2), alpha);
-      tl = (beta - alpha) / beta;
-      scal = 1.0 / (alpha - beta);
-    }
-    double zq[CL];
-#pragma unroll
-    for (int q = 0; q < CL; ++q) {
-      const int c = lane + 64 * q;
-      zq[q] = (c > j && c < s) ? ys[c] + scal * zs[c] : 0.0;
-    }
-#pragma unroll
-    for (int sl = 0; sl < RW; ++sl) {
-      if (rid[sl] <= j) continue;
-      const double u = xi[sl] * scal;
-      if (lane == 0) X[size_t(rid[sl]) * s + j] = u;
-      const double f = tl * u;
-#pragma unroll
-      for (int q = 0; q < CL; ++q) row[sl][q] -= f * zq[q];
-    }
-    if (g == 0 && tid == 0) {
-      d[j] = beta;
-      tauL[j] = tl;
-      X[size_t(j) * s + j] = beta;
-      finite = finite && isfinite(beta);
-    }
-    if (j + 1 < s) {
-      // right reflector from row j after the left update
-      double yq[CL];
-      double part = 0.0;
-#pragma unroll
-      for (int q = 0; q < CL; ++q) {
-        const int c = lane + 64 * q;
-        yq[q] = (c > j && c < s) ? ys[c] - tl * zq[q] : 0.0;
-        if (c > j + 1) part += yq[q] * yq[q];
-      }
-      const double sig2r = wave_total(part);
-      const double z1 = ys[j + 1] + scal * zs[j + 1];
-      const double alpha2 = ys[j + 1] - tl * z1;
-      double tr = 0.0, beta2 = alpha2, scal2 = 0.0;
-      if (sig2r != 0.0) {
-        beta2 = -copysign(sqrt(alpha2 * alpha2 + sig2r), alpha2);
-        tr = (beta2 - alpha2) / beta2;
-        scal2 = 1.0 / (alpha2 - beta2);
-      }
-      double vq[CL];
-#pragma unroll
-      for (int q = 0; q < CL; ++q) {
-        const int c = lane + 64 * q;
-        vq[q] = (c == j + 1) ? 1.0 : ((c > j + 1 && c < s) ? yq[q] * scal2 : 0.0);
-      }
-      if (g == 0 && wave == 0) {
-#pragma unroll
-        for (int q = 0; q < CL; ++q) {
-          const int c = lane + 64 * q;
-          if (c > j + 1 && c < s) X[size_t(j) * s + c] = vq[q];
-        }
-        if (lane == 0) {
-          e[j] = beta2;
-          tauR[j] = tr;
-          X[size_t(j) * s + j + 1] = beta2;
-          finite = finite && isfinite(beta2);
-        }
-      }
-      double acc[RW];
-#pragma unroll
-      for (int sl = 0; sl < RW; ++sl) {
-        acc[sl] = 0.0;
-#pragma unroll
-        for (int q = 0; q < CL; ++q) acc[sl] += row[sl][q] * vq[q];
-      }
-      wave_totals<RW>(acc);
-#pragma unroll
-      for (int sl = 0; sl < RW; ++sl) {
-        if (rid[sl] <= j) continue;
-        const double f = tr * acc[sl];
-#pragma unroll
-        for (int q = 0; q < CL; ++q) row[sl][q] -= f * vq[q];
-      }
-    }
-  }
-  if (g == 0 && tid == 0 && !finite) fail[1] = 1u;
-}
-
-struct BidiagPlan {
-  const void* fn;
-  int rows_per_group;  // 4 * RW
-  bool single;
-  bool two = false;    // two-level exchange
-};
-
-// Columns per lane CL = ceil(s / 64) (s <= 1024); rows per wave RW so that the grid holds at most 16
-// workgroups (a plain launch) where the registers allow (RW * CL <= 64 doubles).  Grids of more
-// than 64 workgroups (s > 256 with long rows, and s > 1024) take the two-level exchange.
-BidiagPlan bidiag_plan(int r, int s) {
-  if (s <= 64 && r <= 64) return {reinterpret_cast<const void*>(k_bidiag<1, 16, true>), 64, true};
-  if (s <= 64) return {reinterpret_cast<const void*>(k_bidiag<1, 32, false>), 128, false};
-  if (s <= 128) return {reinterpret_cast<const void*>(k_bidiag<2, 32, false>), 128, false};
-  if (s <= 256) return {reinterpret_cast<const void*>(k_bidiag<4, 16, false>), 64, false};
-  // past 64 workgroups the partial sums go through the two-level exchange
-  if (s <= 512)
-    return r <= 64 * 32 ? BidiagPlan{reinterpret_cast<const void*>(k_bidiag<8, 8, false>), 32, false}
-                        : BidiagPlan{reinterpret_cast<const void*>(k_bidiag<8, 8, false, true>), 32, false, true};
-  if (s <= 1024)
-    return r <= 64 * 16 ? BidiagPlan{reinterpret_cast<const void*>(k_bidiag<16, 4, false>), 16, false}
-                        : BidiagPlan{reinterpret_cast<const void*>(k_bidiag<16, 4, false, true>), 16, false, true};
-  return {reinterpret_cast<const void*>(k_bidiag<32, 2, false, true>), 8, false, true};
-}
 
 // ---------------------------------------------------------------- bisection
 //
@@ -998,59 +678,6 @@ GemmDesc gd(int64_t M, int64_t N, int64_t K, bool ta, bool tb, int64_t lda, int6
 }
 
 }  // namespace
-
-// Every workgroup reads the G partial-sum vectors of each step (G x s doubles), so the
-// step's exchange grows with G^2 over the device; grids above 64 workgroups are not
-// served (the caller takes the Gram-matrix route instead).
-int bidiag_groups(int r, int s) {
-  if (s < 1 || r < s || s > kBidiagMax || r > kBidiagRowsMax) return 0;
-  const BidiagPlan p = bidiag_plan(r, s);
-  const int G = p.single ? 1 : (r + p.rows_per_group - 1) / p.rows_per_group;
-  return G <= (p.two ? 256 : 64) ? G : 0;
-}
-
-bool bidiag_launch(nsmi_ctx* ctx, double* X, int r, int s, double* d, double* e, double* tauL, double* tauR,
-                   SytrdRun& run) {
-  constexpr int kPlainLaunchMax = 16;
-  const int G = bidiag_groups(r, s);
-  if (G == 0) return false;
-  const BidiagPlan p = bidiag_plan(r, s);
-  if (G > kPlainLaunchMax) {
-    int dev = 0, coop = 0, ncu = 0, per_cu = 0;
-    NSMI_HIP(hipGetDevice(&dev));
-    NSMI_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
-    NSMI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    NSMI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, p.fn, 256, 0));
-    if (!coop || per_cu < 1 || G > ncu * per_cu) return false;
-  }
-  const size_t xn = 2 * size_t(s) + 2 * size_t(G) + 2 * size_t(G) * s + (p.two ? 2 * size_t(s) : 0);
-  run.xch.reset(new Scratch(ctx, sizeof(double) * (p.single ? 1 : xn)));
-  run.flags.reset(new Scratch(ctx, 256));
-  unsigned* bar = run.flags->as<unsigned>();
-  unsigned* failp = bar + 32;
-  reduction_flags_reset(ctx, run.flags->as<unsigned>(), G);
-  int rr = r, ss = s;
-  double* xp = run.xch->as<double>();
-  void* args[] = {&X, &rr, &ss, &d, &e, &tauL, &tauR, &xp, &bar, &failp};
-  {
-    // algorithmic work of a Householder bidiagonalisation: 4 s^2 (r - s / 3) flops
-    ProfScope ps(ctx, NSMI_K_FACT_REDUCE, 4.0 * double(s) * s * (double(r) - double(s) / 3.0),
-                 16.0 * double(r) * s);
-    if (G > kPlainLaunchMax) {
-      const hipError_t st = hipLaunchCooperativeKernel(p.fn, dim3(unsigned(G)), dim3(256), args, 0, ctx->stream);
-      if (st != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-      }
-    } else {
-      NSMI_HIP(hipLaunchKernel(p.fn, dim3(unsigned(G)), dim3(256), args, 0, ctx->stream));
-    }
-  }
-  run.host_flags = static_cast<unsigned*>(stage_take(ctx, 2 * sizeof(unsigned)));
-  run.host_flags[0] = run.host_flags[1] = 0u;
-  NSMI_HIP(hipMemcpyAsync(run.host_flags, failp, 2 * sizeof(unsigned), hipMemcpyDeviceToHost, ctx->stream));
-  return true;
-}
 
 void gk_offdiag(nsmi_ctx* ctx, const double* d, const double* e, int s, double* gk) {
   if (s < 1) return;

@@ -1,0 +1,88 @@
+"""The one-launch reductions behind the truncated factorisation at the edges of their plans.
+
+Tolerances: an SVD's backward error is c n eps ||M|| with a small c; n <= 4096 gives
+1e-12, and the measured values are 5e-15.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import networksolvers_amd as ns
+    c = ns.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("m,n", [(32, 31), (33, 32), (65, 64), (129, 63), (257, 64), (2049, 5), (129, 128), (257, 65),
+                                 (1025, 128), (2049, 127), (257, 256), (513, 129), (1025, 256), (513, 512),
+                                 (600, 512), (2049, 513), (1025, 1025)])
+def test_bidiagonalisation_plan_edges(ctx, m, n):
+    """First shapes past each plan's limits (rows and columns; one workgroup, one XCD with
+    and without sliced columns, all XCDs): M = U C, orthonormal U, the row norms of C the
+    singular values, on both sides."""
+    import networksolvers_amd as ns
+    M = np.random.default_rng(m * 5000 + n).standard_normal((m, n))
+    s = np.linalg.svd(M, compute_uv=False)
+    print(f"bidiagonalisation m={m} n={n}", flush=True)
+    x = ctx.upload(M)
+    for trailing in (False, True):
+        U, C, info = ns.factorize(x, 1, trailing, cutoff=0.0, which_decomp="svd")
+        assert info.route == "svd" and info.kept == n
+        u, c = (U.numpy().T, C.numpy().T) if trailing else (U.numpy(), C.numpy())
+        A = M.T if trailing else M
+        assert np.linalg.norm(u @ c - A) < 1e-12 * np.linalg.norm(M)
+        assert np.abs(u.T @ u - np.eye(n)).max() < 1e-12
+        assert np.abs(np.linalg.norm(c, axis=1) - s).max() < 1e-12 * s[0]
+
+
+def test_bidiagonalisation_of_special_matrices(ctx):
+    """Zero and rank-one matrices, and entries whose squares are near the ends of the range:
+    finite results, orthonormal U, the rank-one matrix reproduced."""
+    import networksolvers_amd as ns
+    rng = np.random.default_rng(11)
+    for m, n in ((40, 40), (150, 130), (300, 280)):
+        one = np.outer(rng.standard_normal(m), rng.standard_normal(n))
+        for name, M in (("zero", np.zeros((m, n))), ("rank one", one), ("small", 1e-146 * rng.standard_normal((m, n))),
+                        ("large", 1e145 * rng.standard_normal((m, n)))):
+            print(f"special {name} m={m} n={n}", flush=True)
+            U, C, info = ns.factorize(ctx.upload(M), 1, False, cutoff=0.0, maxdim=7, which_decomp="svd")
+            u, c = U.numpy(), C.numpy()
+            assert np.isfinite(u).all() and np.isfinite(c).all()
+            assert np.abs(u.T @ u - np.eye(info.kept)).max() < 1e-11
+            if name == "rank one":
+                assert np.linalg.norm(u @ c - M) < 1e-12 * np.linalg.norm(M)
+
+
+def test_reductions_on_more_streams_than_places(ctx):
+    """18 contexts (streams) share the 16 places of the one-XCD groups: results equal to
+    the first context's, bit for bit, with all launches in flight from several threads."""
+    import threading
+
+    import networksolvers_amd as ns
+    M = np.random.default_rng(3).standard_normal((150, 140))
+    ctxs = [ns.Context(0) for _ in range(18)]
+    want = ns.factorize(ctx.upload(M), 1, False, cutoff=0.0, maxdim=20, which_decomp="svd")[1].numpy()
+    got, errors = {}, []
+
+    def work(ids):
+        try:
+            for _ in range(3):
+                for i in ids:
+                    got[i] = ns.factorize(ctxs[i].upload(M), 1, False, cutoff=0.0, maxdim=20,
+                                          which_decomp="svd")[1].numpy()
+        except Exception as ex:   # noqa: BLE001
+            errors.append(ex)
+    ts = [threading.Thread(target=work, args=(range(t, 18, 6),)) for t in range(6)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for c in ctxs:
+        c.close()
+    assert not errors
+    for i in range(18):
+        np.testing.assert_array_equal(got[i], want)
