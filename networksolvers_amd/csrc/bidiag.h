@@ -37,8 +37,6 @@
 // the exchange two steps after it is finished, by blocks of 64 (lo below), so that the
 // buffer rotation's condition holds for every column that still takes part.
 #pragma once
-#include <type_traits>
-
 #include "group.h"
 
 namespace nsmi {
@@ -62,19 +60,6 @@ inline BidiagExchange bidiag_exchange(int cl, int gmax, int groups, bool all) {
   x.ps_words = 3 * sp * x.slots;
   x.words = x.ps_words + 3 * sp * (2 + (all ? 3 * kXcds : 0));
   return x;
-}
-
-// Runs block(CA) for the column blocks from CL down, CA the number of blocks held by the
-// registers it works on (a multiple of STEP): fewer as the matrix shrinks, every register
-// index a constant.
-template <int CA, int STEP, class F>
-__device__ __forceinline__ bool bidiag_blocks(int s, int& cb, const F& block) {
-  while (cb < s && (s - cb + 63) / 64 > CA - STEP) {
-    if (!block(std::integral_constant<int, CA>())) return false;
-    cb += 64;
-  }
-  if constexpr (CA > STEP) return bidiag_blocks<CA - STEP, STEP>(s, cb, block);
-  return true;
 }
 
 template <int CL, int RW, int NW, BidiagMode MODE, int GMAX = 16>
@@ -388,7 +373,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 && (MODE == kOneXcd || MODE == kOn
     }
     return true;
   };
-  if (!bidiag_blocks<CL, STEP>(s, cb, block)) return;
+  if (!column_blocks<CL, STEP>(s, s, cb, block)) return;
   if (lane == 0 && !finite) ctl[kCtlNonFinite] = 1u;
 }
 

@@ -80,8 +80,8 @@ BidiagPlan plan_of() {
 // Measured on gfx950 (us per column; the barrier form with 32-row workgroups spread over
 // the XCDs that these plans replaced: 7.1 at 384 x 384, 17.5 at 1024 x 1024, 28.6 at
 // 2048 x 2048):
-//   one workgroup: 1.4 at 32 x 32 (4 rows per wave), 1.95 at 64 x 64 (8 rows); 3.7 at 128 x
-//   128, against 1.8 on 16 workgroups of one XCD;
+//   one workgroup: 1.4 at 32 x 32 (1.7 on 8 workgroups), 1.95 at 64 x 64 (1.7 on 8
+//   workgroups of one XCD), 3.7 at 128 x 128 (1.8 on 16);
 //   one XCD, everyone reading everyone's sums: 1.9 at 128 x 60, 1.8 at 128 x 128, 2.1 at 256 x
 //   128; 2.26 at 256 x 256 against 2.21 with the columns sliced, 4.0 against 2.5 at 422 x 394;
 //   one XCD, sliced, as few rows per workgroup as 32 workgroups allow: 2.6 at 512 x 512 (3.0
@@ -93,7 +93,7 @@ BidiagPlan plan_of() {
 BidiagPlan bidiag_plan(int r, int s) {
   if (s <= 64) {
     if (r <= 32) return plan_of<1, 4, 8, kOneGroup, 1>();
-    if (r <= 64) return plan_of<1, 8, 8, kOneGroup, 1>();
+    if (r <= 64) return plan_of<1, 2, 4, kOneXcd, 8>();
     if (r <= 128) return plan_of<1, 4, 4, kOneXcd, 8>();
     if (r <= 256) return plan_of<1, 4, 8, kOneXcd, 8>();
     if (r <= 2048) return plan_of<1, 8, 8, kOneXcdSliced, 32>();

@@ -145,13 +145,6 @@ void stage_reset(nsmi_ctx* ctx) {
 
 void stage_done(nsmi_ctx* ctx) { ctx->h_stage_busy = false; }
 
-void reduction_flags_reset(nsmi_ctx* ctx, unsigned* flags, int G) {
-  NSMI_HIP(hipMemsetAsync(flags, 0, 256, ctx->stream));
-  if (G > 1 && ctx->inject_timeouts > 0) {
-    --ctx->inject_timeouts;
-    NSMI_HIP(hipMemsetD32Async(reinterpret_cast<hipDeviceptr_t>(flags + 32), 1, 1, ctx->stream));
-  }
-}
 void scratch_release(nsmi_ctx* ctx, void* p) {
   if (ctx->defer_release)
     ctx->deferred.push_back(p);

@@ -1,381 +1,38 @@
-// Symmetric tridiagonalisation of the truncation's Gram matrix rho (n x n) in one
-// cooperative launch (the eigensolver behind inserter.jl:23 -> ITensors
-// eigen/svd -> LAPACK syevd).  rocSOLVER's blocked sytrd issues about ten small
-// kernels per column and is launch-latency bound at the sizes a sweep produces
-// (about 17 us per column on gfx950 for n <= 2048); here a column costs one grid
-// barrier and a few microseconds of register-resident work.
-//
-// Householder reduction with LAPACK dsytd2 "lower" semantics on the column-major
-// view (rho is symmetric, so the row-major buffer is the same matrix):
-//   for j = 0 .. n-2:  x = A(j+1:n, j);  alpha = x_0, sigma^2 = |x_1:|^2
-//     sigma^2 == 0:    tau_j = 0, e_j = alpha
-//     else:            beta = -sign(alpha) sqrt(alpha^2 + sigma^2), tau_j = (beta - alpha)/beta,
-//                      v = [1, x_1:/(alpha - beta)], e_j = beta
-//     p = tau_j A22 v,  w = p - (tau_j/2)(p.v) v,  A22 -= v w^T + w v^T,  d_j = A(j, j)
-// The output has LAPACK's layout -- d, e, tau, and in the lower triangle of the
-// column-major view the diagonal d, the subdiagonal e and v_j(2:) in A(j+2:n, j)
-// -- which rocsolver_dstedc and the back-transformation apply_q_lower consume.
-//
-// Distribution: workgroup g owns the rows i = g (mod G); row i sits in registers
-// (of one wave, or of one 16-lane group; see the two kernels).  Step j:
-//   1. every workgroup forms v from the column x_j (kept in LDS by all of them);
-//   2. each wave computes p_i = tau v.row_i for its rows i > j and publishes it;
-//      the owner of row j+1 publishes that row (= column j+1, pre-update) as Y;
-//   3. grid barrier;
-//   4. every workgroup reads p and Y, forms w, its own copy of the next column
-//      x_{j+1} = Y - v w_{j+1} - w v_{j+1} and d_{j+1} = Y_{j+1} - 2 w_{j+1},
-//      and applies the rank-2 update to the rows it owns.
-// so one barrier per column suffices.  The exchange buffers alternate by the
-// parity of j: a workgroup writes step j+1's values only after passing barrier j
-// and before barrier j+1, when every workgroup has finished reading step j-1's.
-// Barrier spins are bounded: a workgroup that waits too long raises a flag and
-// leaves, every other one leaves at its next barrier once it sees the flag, so
-// the grid always drains; the host then reports the failure.  fail[0] is that
-// flag; fail[1] is raised when an entry of d or e is NaN or Inf (no barrier or
-// loop bound depends on the values, so such input runs the fixed step count).
+// Symmetric tridiagonalisation of the truncation's Gram matrix rho (n x n) in one launch
+// (the eigensolver behind inserter.jl:23 -> ITensors eigen/svd -> LAPACK syevd): the
+// kernel is k_sytrd (sytrd.h), its plans and launch below; the batched Jacobi solver for
+// small Gram matrices; and the compact-WY back-transformation of the kept vectors.
 #include "internal.h"
+#include "sytrd.h"
 #include "wave.h"
 
 namespace nsmi {
 namespace {
 
-constexpr int kTriThreads = 256;
-
-// Sum over each 16-lane row of the wave (quad permutes, half-row and row mirror)
-// for R values at once; every lane of a row gets its row's total.
-template <int R>
-__device__ inline void row16_totals(double (&a)[R]) {
-#pragma unroll
-  for (int s = 0; s < R; ++s) a[s] += dpp_mov<0xB1, 0xF>(a[s]);  // quad_perm [1,0,3,2]
-#pragma unroll
-  for (int s = 0; s < R; ++s) a[s] += dpp_mov<0x4E, 0xF>(a[s]);  // quad_perm [2,3,0,1]
-#pragma unroll
-  for (int s = 0; s < R; ++s) a[s] += dpp_mov<0x141, 0xF>(a[s]);  // row_half_mirror
-#pragma unroll
-  for (int s = 0; s < R; ++s) a[s] += dpp_mov<0x140, 0xF>(a[s]);  // row_mirror
-}
-
-// Row-group layout (the form for one workgroup, n <= 64, where a wave would
-// otherwise own up to 32 rows and their 6-stage reductions): the 256 threads form
-// 16 groups of 16 lanes (DPP rows); group rg of
-// workgroup g owns the matrix rows (r 16 + rg) G + g, r < RS, in registers, its
-// lane l holding columns l + 16c, c < CC (NP = 16 CC >= n).  So a row's dot
-// product with v is a 16-lane reduction.  v and w live in LDS, double-buffered by
-// the parity of j (a fast wave may write step j+1's v while a slow one still
-// updates with step j's); x_j lives in LDS too.  SINGLE: one workgroup (G == 1),
-// the p / Y exchange in LDS and the barrier a workgroup barrier; otherwise xch
-// holds 4 n doubles of global exchange (P[2][n], Y[2][n]); bar, fail: zero on entry.
-template <int CC, int RS, bool SINGLE>
-__global__ __launch_bounds__(kTriThreads) void k_sytrd_grp(double* __restrict__ A, int n, double* __restrict__ d,
-                                                           double* __restrict__ e, double* __restrict__ tau,
-                                                           double* __restrict__ xch, unsigned* bar,
-                                                           unsigned* fail) {
-  constexpr int NP = 16 * CC;  // padded vector length (a multiple of 64)
-  constexpr int NQ = NP / 64;  // entries per lane of a wave-wide vector pass
-  __shared__ double vs[2][NP], ws[2][NP], xs[NP];
-  __shared__ double xl[SINGLE ? 4 * NP : 1];
-  __shared__ int s_ok;
-  const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int rg = tid >> 4, l16 = tid & 15;
-  double* const xbase = SINGLE ? xl : xch;
-  const int xn = SINGLE ? NP : n;  // stride of the exchange halves
-
-  double row[RS][CC];
-  int rid[RS];
-#pragma unroll
-  for (int r = 0; r < RS; ++r) {
-    const int i = (r * 16 + rg) * G + g;
-    rid[r] = i < n ? i : -1;
-#pragma unroll
-    for (int c = 0; c < CC; ++c) {
-      const int k = l16 + 16 * c;
-      row[r][c] = (i < n && k < n) ? A[size_t(i) * n + k] : 0.0;
-    }
-  }
-  // x_0 = column 0 = row 0 (symmetric); nobody writes A before the first barrier
-  for (int k = tid; k < NP; k += kTriThreads) xs[k] = (k >= 1 && k < n) ? A[k] : 0.0;
-  if (g == 0 && tid == 0) d[0] = A[0];
-  bool finite = isfinite(A[0]);  // of d and e, kept by the thread that writes them
-  __syncthreads();
-
-  unsigned nbar = 0;
-  for (int j = 0; j + 1 < n; ++j) {
-    double* const vb = vs[j & 1];
-    double* const wb = ws[j & 1];
-    double* const P = xbase + (j & 1) * xn;
-    double* const Y = xbase + 2 * xn + (j & 1) * xn;
-    // 1. reflector from x = xs[j+1 ..] (every wave reduces the whole vector)
-    double part = 0.0;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const int k = lane + 64 * q;
-      if (k >= j + 2) part += xs[k] * xs[k];
-    }
-    const double sigma2 = wave_total(part);
-    const double alpha = xs[j + 1];
-    double t = 0.0, beta = alpha, scal = 0.0;
-    if (sigma2 != 0.0) {
-      beta = -copysign(sqrt(alpha * alpha + sigma2), alpha);
-      t = (beta - alpha) / beta;
-      scal = 1.0 / (alpha - beta);
-    }
-    for (int k = tid; k < NP; k += kTriThreads) vb[k] = (k == j + 1) ? 1.0 : (k >= j + 2 ? xs[k] * scal : 0.0);
-    __syncthreads();
-    // 2. p_i = tau v . row_i for own rows i > j; the owner of row j+1 publishes it as Y
-    double acc[RS];
-#pragma unroll
-    for (int r = 0; r < RS; ++r) {
-      acc[r] = 0.0;
-#pragma unroll
-      for (int c = 0; c < CC; ++c)
-        if (16 * c + 15 > j) acc[r] += row[r][c] * vb[l16 + 16 * c];
-    }
-    row16_totals<RS>(acc);
-#pragma unroll
-    for (int r = 0; r < RS; ++r) {
-      if (rid[r] <= j) continue;  // uniform per 16-lane group (rid < 0: empty slot)
-      if (l16 == 0) P[rid[r]] = t * acc[r];
-      if (rid[r] == j + 1) {
-#pragma unroll
-        for (int c = 0; c < CC; ++c) {
-          const int k = l16 + 16 * c;
-          if (k > j && k < n) Y[k] = row[r][c];
-        }
-      }
-    }
-    // 3.
-    if (SINGLE) {
-      __syncthreads();
-    } else if (!grid_barrier(bar, unsigned(G), ++nbar, fail, &s_ok)) {
-      return;
-    }
-    if (g == 0) {
-      // LAPACK layout of column j (column-major view = row j of the buffer)
-      for (int k = tid; k < NP; k += kTriThreads)
-        if (k >= j + 2 && k < n) A[size_t(j) * n + k] = vb[k];
-      if (tid == 0) {
-        e[j] = beta;
-        tau[j] = t;
-        A[size_t(j) * n + j + 1] = beta;
-        finite = finite && isfinite(beta);
-      }
-    }
-    // 4. w = p - (tau/2)(p.v) v (every wave forms p.v over the whole vector), the
-    // next column x_{j+1} and d_{j+1}; wave w writes the entries lane + 64q, q = w mod 4
-    double pq[NQ];
-    part = 0.0;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const int k = lane + 64 * q;
-      pq[q] = (k > j && k < n) ? P[k] : 0.0;
-      part += pq[q] * vb[k];
-    }
-    const double cc = 0.5 * t * wave_total(part);
-    const double w1 = P[j + 1] - cc;  // w_{j+1}, as v_{j+1} = 1
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      if ((q & 3) != wave) continue;  // uniform per wave
-      const int k = lane + 64 * q;
-      const double wk = pq[q] - cc * vb[k];
-      wb[k] = wk;
-      xs[k] = (k >= j + 2 && k < n) ? Y[k] - vb[k] * w1 - wk : 0.0;
-    }
-    if (g == 0 && tid == 0) {
-      const double dn = Y[j + 1] - 2.0 * w1;
-      d[j + 1] = dn;
-      A[size_t(j + 1) * n + j + 1] = dn;
-      finite = finite && isfinite(dn);
-    }
-    __syncthreads();
-    // 5. rank-2 update of the own rows
-#pragma unroll
-    for (int r = 0; r < RS; ++r) {
-      if (rid[r] <= j) continue;
-      const double vi = vb[rid[r]], wi = wb[rid[r]];
-#pragma unroll
-      for (int c = 0; c < CC; ++c)
-        if (16 * c + 15 > j) {
-          const int k = l16 + 16 * c;
-          row[r][c] -= vi * wb[k] + wi * vb[k];
-        }
-    }
-  }
-  if (g == 0 && tid == 0 && !finite) fail[1] = 1u;
-}
-
-// Wave-owned rows (the form for several workgroups): slot s of wave w holds row
-// (4s + w) G + g, lane l holding the columns l + 64c.
-// CL: 64-column slots per lane (n <= 64 CL); RW: rows per wave (G = ceil(n / (4 RW))).
-// SINGLE: one workgroup (G == 1), the p / Y exchange in LDS and the barrier a
-// workgroup barrier.  xch: 4 n doubles of global exchange (P[2][n], Y[2][n]) when
-// G > 1; bar, fail: zero on entry.
-//
-// Every wave keeps its own register copy of x_j, v and w at its lanes' columns
-// (they are cheap to form redundantly), and a wave-private LDS copy of v and w
-// for the broadcast reads v_i, w_i of its rows; so the only synchronisation of a
-// step is the barrier between publishing p / Y and reading them.
-template <int CL, int RW, bool SINGLE>
-__global__ __launch_bounds__(kTriThreads) void k_sytrd_wave(double* __restrict__ A, int n, double* __restrict__ d,
-                                                            double* __restrict__ e, double* __restrict__ tau,
-                                                            double* __restrict__ xch, unsigned* bar,
-                                                            unsigned* fail) {
-  constexpr int NP = 64 * CL;  // padded vector length
-  __shared__ double vl[4][NP], wl[4][NP];
-  __shared__ double xl[SINGLE ? 4 * NP : 1];
-  __shared__ int s_ok;
-  const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  double* __restrict__ vme = vl[wave];
-  double* __restrict__ wme = wl[wave];
-  double* const xbase = SINGLE ? xl : xch;
-  const int xn = SINGLE ? NP : n;  // stride of the exchange halves
-
-  double row[RW][CL];
-  int rid[RW];
-#pragma unroll
-  for (int s = 0; s < RW; ++s) {
-    const int i = (s * 4 + wave) * G + g;
-    rid[s] = i < n ? i : -1;
-#pragma unroll
-    for (int c = 0; c < CL; ++c) {
-      const int k = lane + 64 * c;
-      row[s][c] = (i < n && k < n) ? A[size_t(i) * n + k] : 0.0;
-    }
-  }
-  // x_0 = column 0 = row 0 (symmetric); nobody writes A before the first barrier
-  double xs[CL];
-#pragma unroll
-  for (int c = 0; c < CL; ++c) {
-    const int k = lane + 64 * c;
-    xs[c] = (k >= 1 && k < n) ? A[k] : 0.0;
-  }
-  double alpha = n > 1 ? A[1] : 0.0;
-  if (g == 0 && tid == 0) d[0] = A[0];
-  bool finite = isfinite(A[0]);  // of d and e, kept by the thread that writes them
-
-  unsigned nbar = 0;
-  for (int j = 0; j + 1 < n; ++j) {
-    double* P = xbase + (j & 1) * xn;
-    double* Y = xbase + 2 * xn + (j & 1) * xn;
-    // 1. reflector from x = x_j[j+1 ..]
-    double part = 0.0;
-#pragma unroll
-    for (int c = 0; c < CL; ++c)
-      if (lane + 64 * c >= j + 2) part += xs[c] * xs[c];
-    const double sigma2 = wave_total(part);
-    double t = 0.0, beta = alpha, scal = 0.0;
-    if (sigma2 != 0.0) {
-      beta = -copysign(sqrt(alpha * alpha + sigma2), alpha);
-      t = (beta - alpha) / beta;
-      scal = 1.0 / (alpha - beta);
-    }
-    double vv[CL];
-#pragma unroll
-    for (int c = 0; c < CL; ++c) {
-      const int k = lane + 64 * c;
-      vv[c] = (k == j + 1) ? 1.0 : (k >= j + 2 ? xs[c] * scal : 0.0);
-      vme[k] = vv[c];
-    }
-    // 2. p_i = tau v . row_i for own rows i > j; the owner of row j+1 publishes it as Y
-    double acc[RW];
-#pragma unroll
-    for (int s = 0; s < RW; ++s) {
-      acc[s] = 0.0;
-#pragma unroll
-      for (int c = 0; c < CL; ++c)
-        if (64 * c + 63 > j) acc[s] += row[s][c] * vv[c];
-    }
-    wave_totals<RW>(acc);
-#pragma unroll
-    for (int s = 0; s < RW; ++s) {
-      if (rid[s] <= j) continue;  // uniform per wave (rid < 0: empty slot)
-      if (lane == 0) P[rid[s]] = t * acc[s];
-      if (rid[s] == j + 1) {
-#pragma unroll
-        for (int c = 0; c < CL; ++c) {
-          const int k = lane + 64 * c;
-          if (k > j && k < n) Y[k] = row[s][c];
-        }
-      }
-    }
-    // 3.
-    if (SINGLE) {
-      __syncthreads();
-    } else if (!grid_barrier(bar, unsigned(G), ++nbar, fail, &s_ok)) {
-      return;
-    }
-    if (g == 0 && wave == 0) {
-      // LAPACK layout of column j (column-major view = row j of the buffer)
-#pragma unroll
-      for (int c = 0; c < CL; ++c) {
-        const int k = lane + 64 * c;
-        if (k >= j + 2 && k < n) A[size_t(j) * n + k] = vv[c];
-      }
-      if (lane == 0) {
-        e[j] = beta;
-        tau[j] = t;
-        A[size_t(j) * n + j + 1] = beta;
-        finite = finite && isfinite(beta);
-      }
-    }
-    // 4. w = p - (tau/2)(p.v) v, the next column and d_{j+1}
-    double ww[CL];
-    part = 0.0;
-#pragma unroll
-    for (int c = 0; c < CL; ++c) {
-      const int k = lane + 64 * c;
-      ww[c] = (k > j && k < n) ? P[k] : 0.0;
-      part += ww[c] * vv[c];
-    }
-    const double cc = 0.5 * t * wave_total(part);
-    const double w1 = P[j + 1] - cc;  // w_{j+1}, as v_{j+1} = 1
-#pragma unroll
-    for (int c = 0; c < CL; ++c) {
-      const int k = lane + 64 * c;
-      ww[c] -= cc * vv[c];
-      wme[k] = ww[c];
-      xs[c] = (k >= j + 2 && k < n) ? Y[k] - vv[c] * w1 - ww[c] : 0.0;
-    }
-    if (g == 0 && tid == 0) {
-      const double dn = Y[j + 1] - 2.0 * w1;
-      d[j + 1] = dn;
-      A[size_t(j + 1) * n + j + 1] = dn;
-      finite = finite && isfinite(dn);
-    }
-    wave_sync_lds();
-    alpha = (j + 2 < n) ? Y[j + 2] - vme[j + 2] * w1 - wme[j + 2] : 0.0;
-#pragma unroll
-    for (int s = 0; s < RW; ++s) {
-      if (rid[s] <= j) continue;
-      const double vi = vme[rid[s]], wi = wme[rid[s]];
-#pragma unroll
-      for (int c = 0; c < CL; ++c)
-        if (64 * c + 63 > j) row[s][c] -= vi * ww[c] + wi * vv[c];
-    }
-  }
-  if (g == 0 && tid == 0 && !finite) fail[1] = 1u;
-}
-
 struct TriPlan {
-  const void* fn;
-  int rows_per_group;
+  const void* fn = nullptr;
+  int cl = 1, threads = 0, rows = 0;  // rows per workgroup
+  bool spread = false;                // over all XCDs
 };
+template <int CL, int RW, int NW, bool SHARED>
+TriPlan tri_plan_of(bool spread = false) {
+  return {reinterpret_cast<const void*>(k_sytrd<CL, RW, NW, SHARED>), CL, 64 * NW, RW * NW, spread};
+}
 
-// Measured on gfx950 (per column, n = 41 .. 512): the row-group form on one
-// workgroup wins up to n = 64 (2.4-2.6 us); above that the wave-owned form on as
-// many workgroups as the plain-launch cap of 16 allows, i.e. the fewest rows per
-// wave: 3.4 us at n <= 128 (4 rows per wave) against 4.6 us on one workgroup, 3.9-4.3
-// us at n <= 256 (4 rows) against 5.1-5.5 us with 16 rows, 5.2-5.5 us at n <= 384
-// (6 rows) against 5.5-5.8 us with 8, 5.7 us at n <= 448 (7 rows) against 5.9 us.
-// Each plan uses the narrowest padded width
-// that covers n.
+// Measured on gfx950 (us per column; the grid-barrier form on up to 16 spread workgroups
+// that these plans replaced: 2.4 at n = 64, 3.4 at 128, 3.9 at 256, 5.2-5.7 at 384-448, 10 at
+// 1000): one row per wave 1.05 at n = 64 (2 rows 1.18, 4 rows 1.48) and 1.19 at 128 (1.31,
+// 1.61); two rows 1.5 at 154 and 1.56 at 256 (four 1.9; the words shared through LDS 1.67);
+// four rows 2.5 at 400 and 512 (two on eight waves 3.3: registers).  Above 512 columns a
+// row takes 16 registers a lane and one XCD's 32 workgroups hold the matrix only with
+// spills (4.8 at 700, 9 at 1000), so the group spreads over all XCDs: 3.3 at 513, 3.7 at
+// 700, 4.3 at 1000.
 TriPlan tri_plan(int n) {
-  if (n <= 64) return {reinterpret_cast<const void*>(k_sytrd_grp<4, 4, true>), 64};
-  if (n <= 128) return {reinterpret_cast<const void*>(k_sytrd_wave<2, 4, false>), 16};
-  if (n <= 256) return {reinterpret_cast<const void*>(k_sytrd_wave<4, 4, false>), 16};
-  if (n <= 384) return {reinterpret_cast<const void*>(k_sytrd_wave<8, 6, false>), 24};
-  if (n <= 448) return {reinterpret_cast<const void*>(k_sytrd_wave<8, 7, false>), 28};
-  if (n <= 512) return {reinterpret_cast<const void*>(k_sytrd_wave<8, 8, false>), 32};
-  return {reinterpret_cast<const void*>(k_sytrd_wave<16, 4, false>), 16};
+  if (n <= 64) return tri_plan_of<1, 1, 4, false>();
+  if (n <= 128) return tri_plan_of<2, 1, 4, false>();
+  if (n <= 256) return tri_plan_of<4, 2, 4, false>();
+  if (n <= 512) return tri_plan_of<8, 4, 4, false>();
+  return tri_plan_of<16, 2, 4, true>(true);
 }
 
 // ---- batched Jacobi eigensolver for small Gram matrices ---------------------
@@ -629,63 +286,59 @@ void apply_q_lower(nsmi_ctx* ctx, const double* rho, const double* tau, int n, d
   apply_reflectors(ctx, vt.as<double>(), tau, m, n, Zr, k);
 }
 
-int sytrd_coop_groups(int n) {
-  if (n < 2 || n > kSytrdCoopMax) return 0;
-  const TriPlan p = tri_plan(n);
-  return (n + p.rows_per_group - 1) / p.rows_per_group;
-}
-
-// A: n x n symmetric on the device (row-major == column-major), overwritten with
-// LAPACK's lower-triangle tridiagonal layout; d (n), e and tau (n - 1) on the
-// device.  sytrd_launch enqueues the reduction on ctx->stream and the copy of its
-// two failure flags into run.host_flags; it returns false, with nothing launched,
-// when n is outside the supported range or the device cannot co-schedule the
-// grid (the caller then uses the library path).  sytrd_check reads the flags
-// once the stream has passed the copy.
+// A: n x n symmetric on the device (row-major == column-major), overwritten with the
+// reflectors as k_sytrd leaves them (LAPACK's lower layout without d and e); d (n), e and
+// tau (n - 1) on the device.  sytrd_launch enqueues the reduction on ctx->stream and the
+// copy of its two failure flags into run.host_flags; it returns false, with nothing
+// launched, when n is outside the supported range or the device cannot co-schedule the
+// grid (the caller then uses the library path).  sytrd_check reads the flags once the
+// stream has passed the copy.
 //
-// Grids of up to kPlainLaunchMax workgroups go out as ordinary launches: a
-// cooperative launch waits for the whole device to drain, which would serialise
-// the independent solves that share the GPU, and so few workgroups (one per CU
-// of 256) are co-resident in practice even beside other concurrent reductions;
-// the bounded barrier spin turns the pathological case into an error, not a
-// hang.  Larger grids use the cooperative launch and its co-residency check.
+// A group on one XCD goes out as an ordinary launch: a cooperative launch waits for the
+// whole device to drain, which would serialise the independent solves that share the
+// GPU; that the group becomes resident rests on its place on the XCD
+// (launch_on_one_xcd), and the bounded polls turn the pathological case into an error,
+// not a hang.  A spread group takes the cooperative launch and its co-residency check.
 bool sytrd_launch(nsmi_ctx* ctx, double* A, int n, double* d, double* e, double* tau, SytrdRun& run) {
-  constexpr int kPlainLaunchMax = 16;
-  const int G = sytrd_coop_groups(n);
-  if (G == 0) return false;
+  if (n < 2 || n > kSytrdMax) return false;
   const TriPlan p = tri_plan(n);
-  if (G > kPlainLaunchMax) {
-    int dev = 0, coop = 0, ncu = 0, per_cu = 0;
-    NSMI_HIP(hipGetDevice(&dev));
-    NSMI_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
-    NSMI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    NSMI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, p.fn, kTriThreads, 0));
+  int G = (n + p.rows - 1) / p.rows;
+  if (p.spread) {
+    int coop = 0, ncu = 0, per_cu = 0;
+    NSMI_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device));
+    NSMI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    NSMI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, p.fn, p.threads, 0));
     if (!coop || per_cu < 1 || G > ncu * per_cu) return false;
   }
-  run.xch.reset(new Scratch(ctx, sizeof(double) * 4 * size_t(n)));
-  run.flags.reset(new Scratch(ctx, 256));
-  unsigned* bar = run.flags->as<unsigned>();
-  unsigned* failp = bar + 32;
-  reduction_flags_reset(ctx, run.flags->as<unsigned>(), G);
-  int nn = n;
+  const size_t words = 6 * 64 * size_t(p.cl);
+  run.xch.reset(new Scratch(ctx, sizeof(double) * words));
+  run.flags.reset(new Scratch(ctx, sizeof(unsigned) * kCtlWords));
+  unsigned* ctl = run.flags->as<unsigned>();
   double* xp = run.xch->as<double>();
-  void* args[] = {&A, &nn, &d, &e, &tau, &xp, &bar, &failp};
+  hipLaunchKernelGGL(k_reduction_init, dim3(unsigned((std::max<size_t>(words, kCtlWords) + 255) / 256)), dim3(256), 0,
+                     ctx->stream, xp, words, size_t(0), 1u, 1u, 1u, ctl, int(kCtlWords), reduction_fail0(ctx, G));
+  NSMI_LAUNCH_CHECK();
+  int nn = n, want = -1;
+  void* args[] = {&A, &nn, &d, &e, &tau, &xp, &ctl, &G, &want};
   {
     ProfScope ps(ctx, NSMI_K_FACT_REDUCE, 4.0 / 3.0 * double(n) * n * n, 16.0 * double(n) * n);
-    if (G > kPlainLaunchMax) {
+    if (p.spread) {
       const hipError_t st =
-          hipLaunchCooperativeKernel(p.fn, dim3(unsigned(G)), dim3(kTriThreads), args, 0, ctx->stream);
+          hipLaunchCooperativeKernel(p.fn, dim3(unsigned(G)), dim3(unsigned(p.threads)), args, 0, ctx->stream);
       if (st != hipSuccess) {
         (void)hipGetLastError();
         return false;
       }
     } else {
-      NSMI_HIP(hipLaunchKernel(p.fn, dim3(unsigned(G)), dim3(kTriThreads), args, 0, ctx->stream));
+      launch_on_one_xcd(ctx, [&](int xcd) {
+        want = xcd;
+        NSMI_HIP(hipLaunchKernel(p.fn, dim3(unsigned(kXcds * G)), dim3(unsigned(p.threads)), args, 0, ctx->stream));
+      });
     }
   }
   run.host_flags = static_cast<unsigned*>(stage_take(ctx, 2 * sizeof(unsigned)));
   run.host_flags[0] = run.host_flags[1] = 0u;
-  NSMI_HIP(hipMemcpyAsync(run.host_flags, failp, 2 * sizeof(unsigned), hipMemcpyDeviceToHost, ctx->stream));
+  NSMI_HIP(hipMemcpyAsync(run.host_flags, ctl + kCtlFail, 2 * sizeof(unsigned), hipMemcpyDeviceToHost, ctx->stream));
   return true;
 }
 

@@ -23,6 +23,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "wave.h"
 
 namespace nsmi {
@@ -173,6 +175,19 @@ __device__ inline bool place_all_xcds(unsigned* ctl, int GW, int* x, int* w, boo
   *local = !(p & (1 << 30));
   *x = (p & ~(1 << 30)) % kXcds;
   *w = (p & ~(1 << 30)) / kXcds;
+  return true;
+}
+
+// Runs block(CA) for the column blocks at cb = 0, 64, ... below stop, CA the number of blocks
+// held by the registers it works on (those from cb to the width, rounded up to a multiple
+// of STEP): fewer as the matrix shrinks, every register index a constant.
+template <int CA, int STEP, class F>
+__device__ __forceinline__ bool column_blocks(int stop, int width, int& cb, const F& block) {
+  while (cb < stop && (width - cb + 63) / 64 > CA - STEP) {
+    if (!block(std::integral_constant<int, CA>())) return false;
+    cb += 64;
+  }
+  if constexpr (CA > STEP) return column_blocks<CA - STEP, STEP>(stop, width, cb, block);
   return true;
 }
 

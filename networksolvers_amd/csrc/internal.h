@@ -422,9 +422,8 @@ void small_sym_eigh(int n, const double* A, double* w, double* V);  // host Jaco
 // ---- tridiagonal reduction (eig.hip) ----------------------------------------
 // Householder reduction of a symmetric n x n device matrix to tridiagonal form in
 // LAPACK's dsytrd "lower" layout (one cooperative launch); false when n is outside
-// [2, kSytrdCoopMax] or the device cannot co-schedule the grid.
-constexpr int kSytrdCoopMax = 1024;
-int sytrd_coop_groups(int n);
+// [2, kSytrdMax] or the device cannot co-schedule the grid.
+constexpr int kSytrdMax = 1024;
 // one asynchronous tridiagonal reduction: its exchange and flag buffers, and the
 // host copy of the two failure flags (barrier time-out, non-finite d or e)
 struct SytrdRun {
@@ -432,9 +431,6 @@ struct SytrdRun {
   unsigned* host_flags = nullptr;  // two flags in pinned stage memory
 };
 bool sytrd_launch(nsmi_ctx* ctx, double* A, int n, double* d, double* e, double* tau, SytrdRun& run);
-// zeroes a reduction's barrier and flag words (256 bytes); raises the timeout flag
-// (word 32) when the context has an injected timeout pending and the grid has G > 1
-void reduction_flags_reset(nsmi_ctx* ctx, unsigned* flags, int G);
 // runs launch(xcd) for a kernel whose group of at most 32 workgroups (two of them to a CU)
 // runs on one XCD: the stream's place among the XCDs, see bidiag.hip
 void launch_on_one_xcd(nsmi_ctx* ctx, const std::function<void(int)>& launch);

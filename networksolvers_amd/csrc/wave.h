@@ -1,6 +1,5 @@
-// Wave-level and grid-level helpers shared by the one-launch factorisation
-// kernels (eig.hip, svd.hip): DPP sums of doubles across a 64-lane wave, lane
-// broadcasts, and the bounded grid barrier.
+// Wave-level helpers shared by the factorisation and Krylov kernels: DPP sums of doubles
+// across a 64-lane wave, lane broadcasts.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -54,40 +53,6 @@ __device__ inline void wave_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Grid-wide barrier number n (1, 2, ...) on a monotone arrival counter (target G n).
-// After the workgroup barrier (every wave's writes complete), thread 0 arrives with an
-// agent-scope release add (publishing the workgroup's writes), polls the counter with
-// relaxed agent-scope loads and, once it reads the target, issues one agent-scope
-// acquire fence (the workgroup's later reads then see the other workgroups' writes).
-// Acquire loads in the poll would invalidate the cache on every poll: measured 13%
-// slower per column at 256 workgroups; arrival through per-group counters (16
-// workgroups each, the last arrival of a group adding to the top counter) was slower
-// again (a second dependent atomic).  The spin gives up after a bounded number of
-// polls or when another workgroup has raised the failure flag.
-__device__ inline bool grid_barrier(unsigned* bar, unsigned G, unsigned n, unsigned* fail, int* s_ok) {
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const unsigned target = G * n;
-    __hip_atomic_fetch_add(bar, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-    int ok = 1;
-    for (unsigned spins = 0; __hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target; ++spins) {
-      if ((spins & 255u) == 255u && __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
-        ok = 0;
-        break;
-      }
-      if (spins > (1u << 22)) {
-        atomicOr(fail, 1u);
-        ok = 0;
-        break;
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    *s_ok = ok;
-  }
-  __syncthreads();
-  return *s_ok != 0;
 }
 
 __device__ inline double lane_bcast(double v, int lane) {

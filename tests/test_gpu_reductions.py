@@ -39,6 +39,25 @@ def test_bidiagonalisation_plan_edges(ctx, m, n):
         assert np.abs(np.linalg.norm(c, axis=1) - s).max() < 1e-12 * s[0]
 
 
+@pytest.mark.parametrize("n", [41, 64, 65, 100, 128, 129, 192, 256, 257, 385, 512, 513, 1000, 1024])
+def test_tridiagonalisation_plan_edges(ctx, n):
+    """The eigen route at the edges of the tridiagonalisation's plans, on a matrix with
+    well-separated squares: the kept eigenvalues, orthonormal U, C = U^T M, and each
+    column an eigenvector of the Gram matrix to n eps of its norm."""
+    import networksolvers_amd as ns
+    M = np.random.default_rng(n).standard_normal((n, n + 3))
+    k = n // 2
+    print(f"tridiagonalisation n={n}", flush=True)
+    U, C, info = ns.factorize(ctx.upload(M), 1, False, cutoff=0.0, maxdim=k, which_decomp="eigen")
+    u, c = U.numpy(), C.numpy()
+    s = np.linalg.svd(M, compute_uv=False)
+    assert info.route == "eigen" and info.kept == k
+    assert np.abs(u.T @ u - np.eye(k)).max() < 1e-12
+    assert np.linalg.norm(u.T @ M - c) < 1e-12 * np.linalg.norm(M)
+    assert np.abs(np.linalg.norm(c, axis=1) - s[:k]).max() < 1e-12 * s[0]
+    assert np.abs(M @ (M.T @ u) - u * s[:k] ** 2).max() < 1e-12 * s[0] ** 2
+
+
 def test_bidiagonalisation_of_special_matrices(ctx):
     """Zero and rank-one matrices, and entries whose squares are near the ends of the range:
     finite results, orthonormal U, the rank-one matrix reproduced."""
