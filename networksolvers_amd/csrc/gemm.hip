@@ -3,8 +3,13 @@
 //
 // FP64 / FP32: v_mfma_{f64,f32}_16x16x4 -- 4 waves (2x2; 8 waves as 2x4 for the
 // 128 x 128 tile), each wave owns a sub-tile built from 16x16 MFMA blocks; K is
-// staged in LDS slabs of 16 (32 for the 32 x 32 tile) with register prefetch of the
-// next slab (double-buffered LDS, one barrier per slab).  Lane layouts of the 16x16x4 instructions:
+// staged in LDS slabs of 16 (32 for the 32 x 32 tile) with register prefetch two slabs
+// ahead (double-buffered LDS, one barrier per slab).  Bound: MFMA issue for large products
+// (the 128 x 128 tile is one workgroup per CU and reaches 66 of the 73 TF/s that a large
+// FP64 library product does; 4096 x 1024 x 5120: 823 -> 635 us, 5120 x 4096 x 1024: 758 ->
+// 661 us with the branch-free loop, the unaligned vector loads, the tile order and the
+// tile rule below); for small ones the latency of a slab (852 x 213 x 1065 in FP32: 37 ->
+// 13.6 us).  Lane layouts of the 16x16x4 instructions:
 //   A operand: lane l holds A[l%16][l/16]    B operand: lane l holds B[l/16][l%16]
 //   D (f32):   lane l, item r holds D[4*(l/16)+r][l%16]
 //   D (f64):   lane l, item r holds D[l/16+4*r][l%16]
@@ -59,13 +64,25 @@ struct GemmArgs {
   T* part;
 };
 
-// XCD-aware tile order: consecutive workgroup ids are dealt round-robin to the
-// 8 XCDs, so remap them such that each XCD works on a contiguous band of tiles
-// (neighbouring tiles share A rows / B columns in that XCD's L2).
+// XCD-aware tile order: consecutive workgroup ids are dealt round-robin to the 8 XCDs, so
+// remap them such that each XCD works on a contiguous band of tiles (the first nwg % 8
+// XCDs take one tile more).
 __device__ inline int xcd_remap(int wg, int nwg) {
   constexpr int kXcd = 8;
-  if (nwg < 2 * kXcd || (nwg % kXcd) != 0) return wg;
-  return (wg % kXcd) * (nwg / kXcd) + wg / kXcd;
+  const int xcd = wg % kXcd;
+  return xcd * (nwg / kXcd) + min(xcd, nwg % kXcd) + wg / kXcd;
+}
+// The band walks blocks of 8 tile rows column by column, so that the tiles an XCD
+// has in flight (32 or 64) share as many A rows as B columns in its L2; row by row, each
+// tile row read all of B again (5120 x 4096 x 1024: 669 -> 661 us; 32 x 32 tiles, 73 -> 58
+// us at 2130 x 639 x 852 transposed).
+__device__ inline void tile_of(int tile, int tiles_m, int tiles_n, int& tm, int& tn) {
+  constexpr int kTileRows = 8;
+  const int grp = min(kTileRows, tiles_m) * tiles_n;  // at most the launch's workgroups
+  const int gi = tile / grp, rest = tile % grp;
+  const int gh = min(kTileRows, tiles_m - gi * kTileRows);
+  tm = gi * kTileRows + rest % gh;
+  tn = rest / gh;
 }
 
 // Staging of one operand (X = A, rows m; or B, rows n): KC when X is K-contiguous in
@@ -78,8 +95,16 @@ __device__ inline int xcd_remap(int wg, int nwg) {
 // A and B use the same one), so a lane's BK / 4 values for the slab are contiguous.
 // Otherwise the slab is [BK][R + 4] (row contiguous) and a fragment is one element
 // per k-step at row kl * (BK / 4) + ks.  Each thread copies E consecutive elements of
-// the slab (along k when KC, along the row otherwise); on a slab entirely inside the
-// matrix whose rows start 16-byte aligned, with 16-byte vector loads.
+// the slab (along k when KC, along the row otherwise) with 16-byte loads; these need only
+// the element's alignment, so odd leading dimensions take them too (a quarter of the
+// loads of the element-wise form that such matrices took before, which also tested every
+// element's bounds).  A row past the matrix reads the last row instead: it reaches only
+// rows (columns) of C that are not written.  Only a slab past K's end (the last) and, for
+// a row-contiguous operand, a tile past the last row go element by element.
+template <typename T>
+struct Vec16 {  // 16 bytes at element alignment
+  typedef T type __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
+};
 template <typename T, typename TM, int R, int BK, int NT, bool KC>
 struct Stage {
   static constexpr int E = R * BK / NT;
@@ -99,37 +124,57 @@ struct Stage {
       r = e % R;
     }
   }
-  // global loads of the run into registers; X(row, k) = KC ? X[row * ld + k] : X[k * ld + row]
-  __device__ static void load(const TM* __restrict__ X, int64_t ld, int64_t r0, int64_t k0, int64_t rows,
-                              int64_t kend, bool vec, T (&reg)[E]) {
+  // the run's place in X, X(row, k) = KC ? X[row * ld + k] : X[k * ld + row]: its address at
+  // slab 0 and the step from slab to slab
+  struct Src {
+    const TM* p;
+    int64_t step, gr, gk;
+  };
+  __device__ static Src source(const TM* __restrict__ X, int64_t ld, int64_t r0, int64_t k0, int64_t rows) {
     int r, k;
     run(threadIdx.x, r, k);
-    const int64_t gr = r0 + r, gk = k0 + k;
-    if (vec) {
-      const TM* p = KC ? X + gr * ld + gk : X + gk * ld + gr;
+    Src s;
+    s.gr = KC ? min(r0 + r, rows - 1) : r0 + r;
+    s.gk = k0 + k;
+    s.p = KC ? X + s.gr * ld + s.gk : X + s.gk * ld + s.gr;
+    s.step = KC ? BK : BK * ld;
+    return s;
+  }
+  // slab kt entirely inside K; INR: the run's rows are inside (always when KC)
+  template <bool INR>
+  __device__ static void load(const Src& s, int64_t kt, int64_t rows, T (&reg)[E]) {
+    const TM* const p = s.p + kt * s.step;
+    if constexpr (KC || INR) {
       constexpr int V = 16 / int(sizeof(TM));
       static_assert(E % V == 0, "run length");
 #pragma unroll
       for (int v = 0; v < E / V; ++v) {
-        if constexpr (sizeof(TM) == 8) {
-          const double2 q = *reinterpret_cast<const double2*>(p + v * V);
-          reg[v * V] = T(q.x);
-          reg[v * V + 1] = T(q.y);
-        } else {
-          const float4 q = *reinterpret_cast<const float4*>(p + v * V);
-          reg[v * V] = T(q.x);
-          reg[v * V + 1] = T(q.y);
-          reg[v * V + 2] = T(q.z);
-          reg[v * V + 3] = T(q.w);
-        }
+        const typename Vec16<TM>::type q = *reinterpret_cast<const typename Vec16<TM>::type*>(p + v * V);
+#pragma unroll
+        for (int j = 0; j < V; ++j) reg[v * V + j] = T(q[j]);
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < E; ++j) {
-        const int64_t rr = KC ? gr : gr + j, kk = KC ? gk + j : gk;
-        reg[j] = (rr < rows && kk < kend) ? T(KC ? X[rr * ld + kk] : X[kk * ld + rr]) : T(0);
-      }
+      for (int j = 0; j < E; ++j) reg[j] = T(p[min(s.gr + j, rows - 1) - s.gr]);
     }
+  }
+  // the slab that K ends in (kt * BK + the first slab's k < kend): its elements as they are
+  // stored, those past the end repeat the last one; store_last puts zeros there
+  __device__ static void load_last(const Src& s, int64_t kt, int64_t rows, int64_t kend, int64_t ld, TM (&raw)[E]) {
+    const int64_t k = s.gk + kt * BK;
+    const TM* const base = s.p + kt * s.step;
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      const int64_t kc = min(KC ? k + j : k, kend - 1);
+      raw[j] = KC ? base[kc - k] : base[(kc - k) * ld + (min(s.gr + j, rows - 1) - s.gr)];
+    }
+  }
+  __device__ static void store_last(T* __restrict__ sh, const Src& s, int64_t kt, int64_t kend, const TM (&raw)[E]) {
+    const int64_t k = s.gk + kt * BK;
+    T reg[E];
+#pragma unroll
+    for (int j = 0; j < E; ++j) reg[j] = (KC ? k + j : k) < kend ? T(raw[j]) : T(0);
+    store(sh, reg);
   }
   __device__ static void store(T* __restrict__ s, const T (&reg)[E]) {
     int r, k;
@@ -161,7 +206,8 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_mfma(GemmArgs<T, TBm, TCm> g) 
   const int wm = wave / GN, wn = wave % GN;
   const int nwg = g.tiles_m * g.tiles_n;
   const int tile = xcd_remap(blockIdx.x, nwg);
-  const int tm = tile / g.tiles_n, tn = tile % g.tiles_n;
+  int tm, tn;
+  tile_of(tile, g.tiles_m, g.tiles_n, tm, tn);
   const int64_t m0 = int64_t(tm) * BM, n0 = int64_t(tn) * BN;
   const int64_t bz = blockIdx.z;
   const int64_t kb = int64_t(blockIdx.y) * g.kc;
@@ -169,21 +215,8 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_mfma(GemmArgs<T, TBm, TCm> g) 
   const T* __restrict__ A = g.A + bz * g.sA;
   const TBm* __restrict__ B = g.B + bz * g.sB;
   TCm* __restrict__ C = g.C + bz * g.sC;
-  // vector loads: rows start 16-byte aligned (pitch and base) and the slab is inside
-  const bool va = (g.lda * int64_t(sizeof(T))) % 16 == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0;
-  const bool vb = (g.ldb * int64_t(sizeof(TBm))) % 16 == 0 && (reinterpret_cast<uintptr_t>(B) & 15) == 0;
-  const bool in_m = m0 + BM <= g.M, in_n = n0 + BN <= g.N;
-
-  T ra[SA::E], rb[SB::E];
-  auto load = [&](int64_t k0) {
-    const bool in_k = k0 + BK <= ke;
-    SA::load(A, g.lda, m0, k0, g.M, ke, va && in_m && in_k, ra);
-    SB::load(B, g.ldb, n0, k0, g.N, ke, vb && in_n && in_k, rb);
-  };
-  auto store = [&](int buf) {
-    SA::store(sA[buf], ra);
-    SB::store(sB[buf], rb);
-  };
+  const auto src_a = SA::source(A, g.lda, m0, kb, g.M);
+  const auto src_b = SB::source(B, g.ldb, n0, kb, g.N);
 
   AccT acc[FM][FN];
 #pragma unroll
@@ -191,14 +224,8 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_mfma(GemmArgs<T, TBm, TCm> g) 
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = AccT{0, 0, 0, 0};
 
-  const int64_t nk = (ke - kb + BK - 1) / BK;
-  load(kb);
-  store(0);
-  __syncthreads();
   const int kl = lane >> 4, ml = lane & 15;
-  for (int64_t kt = 0; kt < nk; ++kt) {
-    const int buf = int(kt & 1);
-    if (kt + 1 < nk) load(kb + (kt + 1) * BK);
+  const auto mma = [&](int buf) {
     // the slab's fragments: lane (ml, kl) at k-step ks holds k = kl * KS + ks
     T af[FM][KS], bf[FN][KS];
 #pragma unroll
@@ -219,8 +246,67 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_mfma(GemmArgs<T, TBm, TCm> g) 
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = mfma16(af[i][ks], bf[j][ks], acc[i][j]);
-    if (kt + 1 < nk) store(buf ^ 1);
+  };
+  const int64_t nfull = (ke - kb) / BK;  // slabs entirely inside K
+  // The whole slabs, loads two slabs ahead (two register sets, two LDS buffers, one barrier
+  // per slab).  Past the end the slab index stays at the last one: those loads and
+  // stores land in registers and buffers that no later step uses, and the loop has no
+  // branches.  The slab that K ends in is loaded with the first ones: loaded after the loop it
+  // cost a small product one more round trip (1.5 of 20 us for an environment update at
+  // bonds of 20).
+  const bool tail = nfull * BK < ke - kb;
+  T tail_a[SA::E];
+  TBm tail_b[SB::E];
+  const auto load_tail = [&]() {
+    if (tail) {
+      SA::load_last(src_a, nfull, g.M, ke, g.lda, tail_a);
+      SB::load_last(src_b, nfull, g.N, ke, g.ldb, tail_b);
+    }
+  };
+  const auto whole = [&](auto in_m, auto in_n) {
+    T ra[2][SA::E], rb[2][SB::E];
+    const auto load = [&](int64_t kt, T (&xa)[SA::E], T (&xb)[SB::E]) {
+      SA::template load<decltype(in_m)::value>(src_a, kt, g.M, xa);
+      SB::template load<decltype(in_n)::value>(src_b, kt, g.N, xb);
+    };
+    const int64_t last = nfull - 1;
+    load(0, ra[0], rb[0]);
+    load_tail();
+    SA::store(sA[0], ra[0]);
+    SB::store(sB[0], rb[0]);
+    load(min(int64_t(1), last), ra[1], rb[1]);
     __syncthreads();
+    const auto step = [&](auto set, int64_t kt) {
+      constexpr int S = decltype(set)::value;
+      load(min(kt + 2, last), ra[S], rb[S]);
+      mma(S);
+      SA::store(sA[S ^ 1], ra[S ^ 1]);
+      SB::store(sB[S ^ 1], rb[S ^ 1]);
+      __syncthreads();
+    };
+    int64_t kt = 0;
+    for (; kt + 1 < nfull; kt += 2) {
+      step(std::integral_constant<int, 0>{}, kt);
+      step(std::integral_constant<int, 1>{}, kt + 1);
+    }
+    if (kt < nfull) step(std::integral_constant<int, 0>{}, kt);
+  };
+  if (nfull > 0) {
+    using Yes = std::integral_constant<bool, true>;
+    using No = std::integral_constant<bool, false>;
+    const bool in_m = !TA || m0 + BM <= g.M, in_n = TB || n0 + BN <= g.N;
+    if (in_m && in_n)
+      whole(Yes{}, Yes{});
+    else
+      whole(No{}, No{});
+  } else {
+    load_tail();
+  }
+  if (tail) {
+    SA::store_last(sA[0], src_a, nfull, ke, tail_a);
+    SB::store_last(sB[0], src_b, nfull, ke, tail_b);
+    __syncthreads();
+    mma(0);
   }
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -317,18 +403,31 @@ void launch_tile(nsmi_ctx* ctx, const GemmDesc& d, GemmArgs<T, TBm, TCm>& a) {
   }
 }
 
+// whether tiles of TS x TS leave at most a fifth of the last round over the 256 CUs (and of
+// the edge tiles) unused
+template <int TS>
+bool tiles_fill(const GemmDesc& d) {
+  const int64_t tiles = ((d.M + TS - 1) / TS) * ((d.N + TS - 1) / TS) * d.batch;
+  const int64_t rounds = (tiles + 255) / 256;
+  return double(d.M) * double(d.N) * double(d.batch) >= 0.8 * (double(TS) * TS * 256.0) * double(rounds);
+}
+
+// The 128 x 128 tile (one workgroup per CU in FP64) only where its rounds are full: it
+// reaches 66 TF/s at 2048 x 2048 x 1024 (32 x 32: 54-56), loses at 3072 x 3072 x 1024 (75%
+// full: 377 us against 345) and at 1536 x 1536 x 1024 (56%: 127 against 93).  Everywhere
+// else the 32 x 32 tile, whose deep slabs and many workgroups hide the latency: in FP64 it
+// is never behind 64 x 64 by more than the runs differ (1024 x 1024 x 1024: 44 us against
+// 50-55; 1536 x 1536 x 1024: 93 against 115-138), which is therefore not built for FP64.  In
+// FP32 64 x 64 wins from about two full rounds (1536 x 1280 x 1024: 40 us against 45;
+// 2176 x 2176 x 1024: 94 against 108) and loses before (1024 x 1024 x 1024: 26 against 24).
 template <typename T, typename TBm, typename TCm, int ROLE>
 void launch_role(nsmi_ctx* ctx, const GemmDesc& d, GemmArgs<T, TBm, TCm>& a) {
-  // the largest tile that still gives every CU work: 128x128 when that makes >= 2
-  // workgroups per CU, 64x64 when >= 1 per CU, else 32x32 (small bond dimensions)
-  const int64_t big = ((d.M + 127) / 128) * ((d.N + 127) / 128) * d.batch;
-  const int64_t mid = ((d.M + 63) / 64) * ((d.N + 63) / 64) * d.batch;
-  if (big >= 512)
-    launch_tile<T, TBm, TCm, 128, 128, ROLE>(ctx, d, a);
-  else if (mid >= 256)
-    launch_tile<T, TBm, TCm, 64, 64, ROLE>(ctx, d, a);
-  else
-    launch_tile<T, TBm, TCm, 32, 32, ROLE>(ctx, d, a);
+  if (tiles_fill<128>(d)) return launch_tile<T, TBm, TCm, 128, 128, ROLE>(ctx, d, a);
+  if constexpr (sizeof(T) == 4) {
+    const int64_t mid = ((d.M + 63) / 64) * ((d.N + 63) / 64) * d.batch;
+    if (mid >= 448 && tiles_fill<64>(d)) return launch_tile<T, TBm, TCm, 64, 64, ROLE>(ctx, d, a);
+  }
+  launch_tile<T, TBm, TCm, 32, 32, ROLE>(ctx, d, a);
 }
 
 template <typename T>

@@ -1,0 +1,57 @@
+"""The MFMA products at the edges of their tiles and K slabs, through the H_eff apply and the
+environment update, against NumPy in FP64.
+
+The sizes: one element; below, at and past a 16 x 16 block, a 32 x 32 tile and a K slab
+of 16 or 32 (K = chi for the first product, 5 chi for the second); odd leading dimensions
+(odd chi); the 64 x 64 tile of FP32 (1505 x 1268); the 128 x 128 tile, ragged on both
+sides and in K (2105 x 1796 x 421).
+
+Bar: a sum of K rounded products in random signs is off by about sqrt(K) u, three
+contractions follow each other and the inputs are rounded once, so 8 sqrt(K) u with K the
+longest inner dimension (u = 2^-53, 2^-24 in FP32); the largest seen is about a quarter of that.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+DW, D = 5, 2
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import networksolvers_amd as ns
+    c = ns.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("precision,u", [("fp64", 2.0**-53), ("fp32", 2.0**-24)])
+@pytest.mark.parametrize("cl,cr", [(1, 1), (3, 2), (15, 17), (16, 16), (17, 31), (32, 33), (63, 65), (129, 95),
+                                   (301, 317), (421, 449)])
+def test_products_at_tile_edges(ctx, cl, cr, precision, u):
+    import networksolvers_amd as ns
+    rng = np.random.default_rng(cl * 1000 + cr)
+    L, R = rng.standard_normal((cl, DW, cl)), rng.standard_normal((cr, DW, cr))
+    W = rng.standard_normal((DW, DW, D, D))
+    x = rng.standard_normal((cl, D, D, cr))
+    from oracle import chain
+    want = chain.heff2_apply(L, W, W, R, x)
+    H = ns.HeffMap(ctx.upload(L), ctx.upload(W), ctx.upload(W), ctx.upload(R), precision)
+    got = H(ctx.upload(x)).numpy()
+    K = DW * max(cl, cr)
+    assert np.linalg.norm(got - want) <= 8 * np.sqrt(K) * u * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("side", [0, 1])
+@pytest.mark.parametrize("ca,cb", [(1, 3), (15, 17), (31, 65), (95, 129), (451, 449)])
+def test_environment_products_at_tile_edges(ctx, ca, cb, side):
+    import networksolvers_amd as ns
+    from oracle import chain
+    rng = np.random.default_rng(ca * 1000 + cb)
+    A, W = rng.standard_normal((ca, D, cb)), rng.standard_normal((DW, DW, D, D))
+    E = rng.standard_normal((ca, DW, ca) if side == 0 else (cb, DW, cb))
+    want = chain.env_left(E, A, W) if side == 0 else chain.env_right(E, A, W)
+    got = ns.env_update(ctx.upload(E), ctx.upload(A), ctx.upload(W), side).numpy()
+    K = DW * max(ca, cb)
+    assert np.linalg.norm(got - want) <= 8 * np.sqrt(K) * 2.0**-53 * np.linalg.norm(want)
