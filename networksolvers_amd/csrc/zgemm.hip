@@ -3,7 +3,7 @@
 //
 // Complex tensors are interleaved (re, im) pairs.  Tiles are staged into LDS as
 // separate real and imaginary planes (conjugation applied at staging), and each
-// 16x16 output block takes four real MFMAs:
+// 16x16 output block takes four real MFMAs (small grids: k_zgemm_wave, without LDS tiles):
 //   re += ar.br - ai.bi      im += ar.bi + ai.br
 // Row-major, op(A) M x K (A stored K x M when transA), op(B) K x N (stored N x K
 // when transB); C = op(A) op(B) (no scaling).  Output rows of the f64 MFMA are
@@ -194,26 +194,136 @@ __global__ __launch_bounds__(256) void k_zgemm(ZArgs<T> g) {
       }
 }
 
+// The same product for grids too small to fill the chip, where a tile's serial chain of
+// slabs (load, barrier, MFMA) is the whole time: one 16 x 16 block of C per
+// workgroup, K dealt to its 8 waves in chunks of 16, operands straight from memory into
+// the MFMA registers (every element of a block's rows is used once: staging through LDS
+// would add a barrier per slab and share nothing), the next chunk's loads in flight, and
+// the 8 partial sums added in wave order through LDS.
+template <typename T, bool TA, bool TB, int ROLE, int MODE = 0>
+__global__ __launch_bounds__(512) void k_zgemm_wave(ZArgs<T> g) {
+  typedef typename ZT<T>::acc Acc;
+  typedef typename ZT<T>::pair V2;
+  constexpr int NW = 8, U = 4;
+  __shared__ T part[NW][8][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int kl = lane >> 4, ml = lane & 15;
+  const int tile = zxcd_remap(blockIdx.x, g.tiles_m * g.tiles_n);
+  const int64_t m0 = int64_t(tile / g.tiles_n) * 16, n0 = int64_t(tile % g.tiles_n) * 16;
+  // rows and columns past the matrix repeat the last one: they reach only elements of C
+  // that are not written
+  const int64_t am = min(m0 + ml, g.M - 1), bn = min(n0 + ml, g.N - 1);
+  const T sa = g.conjA ? T(-1) : T(1), sb = g.conjB ? T(-1) : T(1);
+  const int64_t nch = (g.K + 4 * U - 1) / (4 * U);
+  const int64_t ar0 = MODE == 1 && g.arow ? g.arow[am] : am * g.lda;
+  V2 a[2][U], b[2][U];
+  const auto load = [&](int64_t c, V2 (&xa)[U], V2 (&xb)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t k = min(c * (4 * U) + u * 4 + kl, g.K - 1);
+      if constexpr (MODE == 1) {
+        const int64_t off = ar0 + (g.arow ? g.acol[k] : k);
+        if (g.a_f64) {
+          const d2 w = *reinterpret_cast<const d2*>(reinterpret_cast<const double*>(g.A) + 2 * off);
+          xa[u] = V2{T(w.x), T(w.y)};
+        } else {
+          xa[u] = *reinterpret_cast<const V2*>(g.A + 2 * off);
+        }
+      } else {
+        xa[u] = *reinterpret_cast<const V2*>(g.A + 2 * (TA ? k * g.lda + am : ar0 + k));
+      }
+      xb[u] = *reinterpret_cast<const V2*>(g.B + 2 * (TB ? bn * g.ldb + k : k * g.ldb + bn));
+    }
+  };
+  Acc acr = Acc{0, 0, 0, 0}, aci = Acc{0, 0, 0, 0};
+  const auto mma = [&](int64_t c, const V2 (&xa)[U], const V2 (&xb)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool in = c * (4 * U) + u * 4 + kl < g.K;
+      const T ar = in ? xa[u].x : T(0), ai = in ? sa * xa[u].y : T(0);
+      const T br = in ? xb[u].x : T(0), bi = in ? sb * xb[u].y : T(0);
+      acr = ZT<T>::mfma(ar, br, acr);
+      aci = ZT<T>::mfma(ar, bi, aci);
+      acr = ZT<T>::mfma(-ai, bi, acr);
+      aci = ZT<T>::mfma(ai, br, aci);
+    }
+  };
+  if (wave < nch) {
+    load(wave, a[0], b[0]);
+    for (int64_t c = wave; c < nch; c += 2 * NW) {
+      load(min(c + NW, nch - 1), a[1], b[1]);
+      mma(c, a[0], b[0]);
+      if (c + NW >= nch) break;
+      load(min(c + 2 * NW, nch - 1), a[0], b[0]);
+      mma(c + NW, a[1], b[1]);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    part[wave][r][lane] = acr[r];
+    part[wave][4 + r][lane] = aci[r];
+  }
+  __syncthreads();
+  if (tid >= 256) return;
+  const int r = wave;  // waves 0..3 write item r of every lane
+  V2 v = {T(0), T(0)};
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    v.x += part[w][r][lane];
+    v.y += part[w][4 + r][lane];
+  }
+  const int64_t gm = m0 + ZT<T>::row(kl, r), gn = n0 + ml;
+  if (gm >= g.M || gn >= g.N) return;
+  if constexpr (MODE == 1) {
+    const int64_t off = g.crow ? g.crow[gm] + g.ccol[gn] : gm * g.ldc + gn;
+    if (g.c_f64)
+      *reinterpret_cast<d2*>(reinterpret_cast<double*>(g.C) + 2 * off) = d2{double(v.x), double(v.y)};
+    else
+      *reinterpret_cast<V2*>(g.C + 2 * off) = v;
+  } else {
+    *reinterpret_cast<V2*>(g.C + 2 * (gm * g.ldc + gn)) = v;
+  }
+}
+
 template <typename T, int BM, int BN, int ROLE>
 void zlaunch(nsmi_ctx* ctx, const GemmDesc& d, ZArgs<T>& a) {
   a.tiles_m = int((d.M + BM - 1) / BM);
   a.tiles_n = int((d.N + BN - 1) / BN);
   dim3 grid(unsigned(a.tiles_m) * unsigned(a.tiles_n));
+#define NSMI_ZGEMM_GO(TA, TB)                                                                  \
+  do {                                                                                         \
+    if constexpr (BM == 16)                                                                    \
+      NSMI_LAUNCH_TIMED(ctx, (k_zgemm_wave<T, TA, TB, ROLE>), grid, dim3(512), a);             \
+    else                                                                                       \
+      NSMI_LAUNCH_TIMED(ctx, (k_zgemm<T, BM, BN, TA, TB, ROLE>), grid, dim3(256), a);          \
+  } while (0)
   if (!d.transA && !d.transB)
-    NSMI_LAUNCH_TIMED(ctx, (k_zgemm<T, BM, BN, false, false, ROLE>), grid, dim3(256), a);
+    NSMI_ZGEMM_GO(false, false);
   else if (!d.transA && d.transB)
-    NSMI_LAUNCH_TIMED(ctx, (k_zgemm<T, BM, BN, false, true, ROLE>), grid, dim3(256), a);
+    NSMI_ZGEMM_GO(false, true);
   else if (d.transA && !d.transB)
-    NSMI_LAUNCH_TIMED(ctx, (k_zgemm<T, BM, BN, true, false, ROLE>), grid, dim3(256), a);
+    NSMI_ZGEMM_GO(true, false);
   else
-    NSMI_LAUNCH_TIMED(ctx, (k_zgemm<T, BM, BN, true, true, ROLE>), grid, dim3(256), a);
+    NSMI_ZGEMM_GO(true, true);
+#undef NSMI_ZGEMM_GO
   NSMI_LAUNCH_CHECK();
+}
+
+// k_zgemm_wave where 32 x 32 tiles leave CUs without one and K is more than one of their
+// slabs.  Measured (M, N, K; us, wave form / 32 x 32): ComplexF64 240, 60, 300: 6.6 / 20.5;
+// 300, 240, 60: 4.4 / 6.7; 800, 200, 1000 (175 tiles): 41 / 62; ComplexF32 400, 100, 500:
+// 7.4 / 24.6.  At 256 tiles (512, 512, 512) it is 31 / 36 and, with B transposed, 40 / 36; beyond
+// it loses (1000, 800, 200: 40-56 / 38), and with K <= 8 both are one round trip (3.3 / 3.1).
+inline bool wave_form(int64_t M, int64_t N, int64_t K) {
+  return K > 8 && ((M + 31) / 32) * ((N + 31) / 32) < 256;
 }
 
 template <typename T, int ROLE>
 void zrole(nsmi_ctx* ctx, const GemmDesc& d, ZArgs<T>& a) {
   const int64_t mid = ((d.M + 63) / 64) * ((d.N + 63) / 64);
-  if (mid >= 256)
+  if (wave_form(d.M, d.N, d.K))
+    zlaunch<T, 16, 16, ROLE>(ctx, d, a);
+  else if (mid >= 256)
     zlaunch<T, 64, 64, ROLE>(ctx, d, a);
   else
     zlaunch<T, 32, 32, ROLE>(ctx, d, a);
@@ -246,7 +356,12 @@ void gemm_net_t(nsmi_ctx* ctx, const ZNetGemm& z) {
   a.a_f64 = z.a_f64 ? 1 : 0;
   a.c_f64 = z.c_f64 ? 1 : 0;
   const int64_t mid = ((z.M + 63) / 64) * ((z.N + 63) / 64);
-  if (mid >= 256) {
+  if (wave_form(z.M, z.N, z.K)) {
+    a.tiles_m = int((z.M + 15) / 16);
+    a.tiles_n = int((z.N + 15) / 16);
+    NSMI_LAUNCH_TIMED(ctx, (k_zgemm_wave<T, false, false, kRoleHeff2, 1>), dim3(unsigned(a.tiles_m) * a.tiles_n),
+                      dim3(512), a);
+  } else if (mid >= 256) {
     a.tiles_m = int((z.M + 63) / 64);
     a.tiles_n = int((z.N + 63) / 64);
     NSMI_LAUNCH_TIMED(ctx, (k_zgemm<T, 64, 64, false, false, kRoleHeff2, 1>), dim3(unsigned(a.tiles_m) * a.tiles_n),

@@ -4,7 +4,9 @@ environment update, against NumPy in FP64.
 The sizes: one element; below, at and past a 16 x 16 block, a 32 x 32 tile and a K slab
 of 16 or 32 (K = chi for the first product, 5 chi for the second); odd leading dimensions
 (odd chi); the 64 x 64 tile of FP32 (1505 x 1268); the 128 x 128 tile, ragged on both
-sides and in K (2105 x 1796 x 421).
+sides and in K (2105 x 1796 x 421).  Complex: K below, at and past the 8 of a slab and the 16
+of a wave's chunk, fewer and more chunks than the 8 waves, and both sides of the rule between
+the forms (252 and 286 tiles of 32 x 32).
 
 Bar: a sum of K rounded products in random signs is off by about sqrt(K) u, three
 contractions follow each other and the inputs are rounded once, so 8 sqrt(K) u with K the
@@ -41,6 +43,39 @@ def test_products_at_tile_edges(ctx, cl, cr, precision, u):
     got = H(ctx.upload(x)).numpy()
     K = DW * max(cl, cr)
     assert np.linalg.norm(got - want) <= 8 * np.sqrt(K) * u * np.linalg.norm(want)
+
+
+def _crand(rng, shape):
+    return rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+
+
+@pytest.mark.parametrize("precision,u", [("fp64", 2.0**-53), ("fp32", 2.0**-24)])
+@pytest.mark.parametrize("cl,cr", [(1, 1), (8, 9), (9, 2), (15, 17), (16, 16), (17, 31), (33, 32), (129, 95), (135, 97)])
+def test_complex_products_at_tile_edges(ctx, cl, cr, precision, u):
+    import networksolvers_amd as ns
+    from oracle import chain
+    rng = np.random.default_rng(cl * 1000 + cr)
+    L, R, W = _crand(rng, (cl, DW, cl)), _crand(rng, (cr, DW, cr)), rng.standard_normal((DW, DW, D, D))
+    x = _crand(rng, (cl, D, D, cr))
+    want = chain.heff2_apply(L, W, W, R, x)
+    H = ns.HeffMap(ctx.upload(L), ctx.upload(W), ctx.upload(W), ctx.upload(R), precision)
+    got = H(ctx.upload(x)).numpy()
+    K = DW * max(cl, cr)
+    assert np.linalg.norm(got - want) <= 8 * np.sqrt(2 * K) * u * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("side", [0, 1])
+@pytest.mark.parametrize("ca,cb", [(1, 9), (8, 16), (17, 15), (31, 65), (129, 95)])
+def test_complex_environment_products_at_tile_edges(ctx, ca, cb, side):
+    import networksolvers_amd as ns
+    from oracle import chain
+    rng = np.random.default_rng(ca * 1000 + cb)
+    A, W = _crand(rng, (ca, D, cb)), rng.standard_normal((DW, DW, D, D))
+    E = _crand(rng, (ca, DW, ca) if side == 0 else (cb, DW, cb))
+    want = chain.env_left(E, A, W) if side == 0 else chain.env_right(E, A, W)
+    got = ns.env_update(ctx.upload(E), ctx.upload(A), ctx.upload(W), side).numpy()
+    K = DW * max(ca, cb)
+    assert np.linalg.norm(got - want) <= 8 * np.sqrt(2 * K) * 2.0**-53 * np.linalg.norm(want)
 
 
 @pytest.mark.parametrize("side", [0, 1])
