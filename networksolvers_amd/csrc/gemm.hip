@@ -341,6 +341,102 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(const T* __restrict__ par
   C[m * ldc + n] = TCm(v);
 }
 
+// The same product for grids too small to fill the chip, where a tile's serial chain of
+// slabs (load, barrier, MFMA) is the whole time: one 16 x 16 block of C per workgroup, K
+// dealt to its 8 waves in chunks of 16 (lane group kl takes k = 4 kl .. 4 kl + 3 of a chunk: 16-byte
+// loads of a K-contiguous operand), operands straight from memory into the MFMA registers
+// (every element of a block's rows is used once: LDS would add a barrier per slab and
+// share nothing), three chunks in flight per wave, and the 8 partial sums added in wave
+// order through LDS.  No partial sums in memory and no second launch, as a split over K has.
+template <typename T, typename TM, bool KC>
+struct WaveOperand {
+  const TM* p;  // element (row, k = 4 kl)
+  int64_t ld, k0;
+  __device__ WaveOperand(const TM* __restrict__ X, int64_t ld_, int64_t row, int kl)
+      : p(KC ? X + row * ld_ + 4 * kl : X + 4 * kl * ld_ + row), ld(ld_), k0(4 * kl) {}
+  __device__ void load(int64_t c, T (&reg)[4]) const {
+    const TM* const q = p + (KC ? c * 16 : c * 16 * ld);
+    if constexpr (KC) {
+      constexpr int V = 16 / int(sizeof(TM));
+#pragma unroll
+      for (int v = 0; v < 4 / V; ++v) {
+        const typename Vec16<TM>::type x = *reinterpret_cast<const typename Vec16<TM>::type*>(q + v * V);
+#pragma unroll
+        for (int j = 0; j < V; ++j) reg[v * V + j] = T(x[j]);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) reg[j] = T(q[j * ld]);
+    }
+  }
+  __device__ void load_last(int64_t c, int64_t K, T (&reg)[4]) const {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int64_t k = c * 16 + k0 + j, kc = min(k, K - 1) - k0;
+      const T v = T(p[KC ? kc : kc * ld]);
+      reg[j] = k < K ? v : T(0);
+    }
+  }
+};
+
+template <typename T, typename TBm, typename TCm, bool TA, bool TB, int ROLE>
+__global__ __launch_bounds__(512) void k_gemm_wave(GemmArgs<T, TBm, TCm> g) {
+  typedef typename Acc<T>::type AccT;
+  constexpr int NW = 8, D = 3;
+  __shared__ T part[NW][4][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int kl = lane >> 4, ml = lane & 15;
+  int tm, tn;
+  tile_of(xcd_remap(blockIdx.x, g.tiles_m * g.tiles_n), g.tiles_m, g.tiles_n, tm, tn);
+  const int64_t m0 = int64_t(tm) * 16, n0 = int64_t(tn) * 16, bz = blockIdx.z;
+  // rows and columns past the matrix repeat the last one: they reach only elements of C
+  // that are not written
+  const WaveOperand<T, T, !TA> oa(g.A + bz * g.sA, g.lda, min(m0 + ml, g.M - 1), kl);
+  const WaveOperand<T, TBm, TB> ob(g.B + bz * g.sB, g.ldb, min(n0 + ml, g.N - 1), kl);
+  AccT acc = AccT{0, 0, 0, 0};
+  const auto mma = [&](const T (&a)[4], const T (&b)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc = mfma16(a[u], b[u], acc);
+  };
+  const int64_t nfull = g.K / 16;
+  T a[D][4], b[D][4];
+  if (wave < nfull) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int64_t c = min(int64_t(wave + d * NW), nfull - 1);
+      oa.load(c, a[d]);
+      ob.load(c, b[d]);
+    }
+  }
+  for (int64_t c0 = wave; c0 < nfull; c0 += D * NW)
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (c0 + d * NW >= nfull) break;
+      mma(a[d], b[d]);
+      const int64_t c = min(c0 + (d + D) * NW, nfull - 1);
+      oa.load(c, a[d]);
+      ob.load(c, b[d]);
+    }
+  if (nfull * 16 < g.K && wave == nfull % NW) {
+    oa.load_last(nfull, g.K, a[0]);
+    ob.load_last(nfull, g.K, b[0]);
+    mma(a[0], b[0]);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) part[wave][r][lane] = acc[r];
+  __syncthreads();
+  if (tid >= 256) return;
+  T sum = T(0);  // waves 0..3 write item r = wave of every lane
+#pragma unroll
+  for (int w = 0; w < NW; ++w) sum += part[w][wave][lane];
+  const int64_t gm = m0 + out_row<T>(kl, wave), gn = n0 + ml;
+  if (gm >= g.M || gn >= g.N) return;
+  TCm* const C = g.C + bz * g.sC;
+  T v = g.alpha * sum;
+  if (g.beta != T(0)) v += g.beta * T(C[gm * g.ldc + gn]);
+  C[gm * g.ldc + gn] = TCm(v);
+}
+
 // number of K splits: only for single products whose tile grid leaves most CUs idle
 // and whose K is long; each split keeps at least four K stages
 template <int BM, int BN>
@@ -403,6 +499,22 @@ void launch_tile(nsmi_ctx* ctx, const GemmDesc& d, GemmArgs<T, TBm, TCm>& a) {
   }
 }
 
+template <typename T, typename TBm, typename TCm, int ROLE>
+void launch_wave(nsmi_ctx* ctx, const GemmDesc& d, GemmArgs<T, TBm, TCm>& a) {
+  a.tiles_m = int((d.M + 15) / 16);
+  a.tiles_n = int((d.N + 15) / 16);
+  const dim3 grid(unsigned(a.tiles_m) * unsigned(a.tiles_n), 1, unsigned(d.batch)), block(512);
+  if (!d.transA && !d.transB)
+    NSMI_LAUNCH_TIMED(ctx, (k_gemm_wave<T, TBm, TCm, false, false, ROLE>), grid, block, a);
+  else if (!d.transA && d.transB)
+    NSMI_LAUNCH_TIMED(ctx, (k_gemm_wave<T, TBm, TCm, false, true, ROLE>), grid, block, a);
+  else if (d.transA && !d.transB)
+    NSMI_LAUNCH_TIMED(ctx, (k_gemm_wave<T, TBm, TCm, true, false, ROLE>), grid, block, a);
+  else
+    NSMI_LAUNCH_TIMED(ctx, (k_gemm_wave<T, TBm, TCm, true, true, ROLE>), grid, block, a);
+  NSMI_LAUNCH_CHECK();
+}
+
 // whether tiles of TS x TS leave at most a fifth of the last round over the 256 CUs (and of
 // the edge tiles) unused
 template <int TS>
@@ -417,11 +529,18 @@ bool tiles_fill(const GemmDesc& d) {
 // full: 377 us against 345) and at 1536 x 1536 x 1024 (56%: 127 against 93).  Everywhere
 // else the 32 x 32 tile, whose deep slabs and many workgroups hide the latency: in FP64 it
 // is never behind 64 x 64 by more than the runs differ (1024 x 1024 x 1024: 44 us against
-// 50-55; 1536 x 1536 x 1024: 93 against 115-138), which is therefore not built for FP64.  In
+// 50-55; 1536 x 1536 x 1024: 93 against 115-138), which is therefore not built for FP64.
+// Up to 64 tiles of 32 x 32 the wave form, while K is short enough for its uncoalesced reads (512
+// in FP64, 1024 in FP32); us, wave form / 32 x 32 with its split: FP64 60, 60, 60: 3.5 / 4.4;
+// 394, 64, 394: 5.5-6.1 / 8.2; 400, 100, 500: 6.5 / 8.7; FP32 64, 64, 1024: 5.4-7.0 / 7.9; 400, 100,
+// 500: 4.4 / 7.6.  It loses at more tiles (FP64 320, 256, 64, 80 tiles: 5.2 / 4.1; 384, 384, 384: 11-18
+// / 8.7) and longer K (FP64 64, 64, 1024: 7.4-11.9 / 9.0; 64, 200, 2048: 11-19 / 10.8).  In
 // FP32 64 x 64 wins from about two full rounds (1536 x 1280 x 1024: 40 us against 45;
 // 2176 x 2176 x 1024: 94 against 108) and loses before (1024 x 1024 x 1024: 26 against 24).
 template <typename T, typename TBm, typename TCm, int ROLE>
 void launch_role(nsmi_ctx* ctx, const GemmDesc& d, GemmArgs<T, TBm, TCm>& a) {
+  if (((d.M + 31) / 32) * ((d.N + 31) / 32) * d.batch <= 64 && d.K <= 4096 / int64_t(sizeof(T)))
+    return launch_wave<T, TBm, TCm, ROLE>(ctx, d, a);
   if (tiles_fill<128>(d)) return launch_tile<T, TBm, TCm, 128, 128, ROLE>(ctx, d, a);
   if constexpr (sizeof(T) == 4) {
     const int64_t mid = ((d.M + 63) / 64) * ((d.N + 63) / 64) * d.batch;
