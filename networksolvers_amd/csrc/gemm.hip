@@ -603,9 +603,8 @@ void gemm_f32_heff2_cd(nsmi_ctx* ctx, const GemmDesc& d, const float* A, const f
 // both operands K-contiguous bf16 planes (row pitch Kp, Kp % 32 == 0, padding
 // zero).  TERMS == 3 computes Ahi.Bhi + Ahi.Blo + Alo.Bhi (bf16x3 split
 // products, FP32 accumulation); TERMS == 1 computes Ahi.Bhi.
-// 512 threads = 8 waves (2 x 4), 128 x 128 tile, K slab 32 (one MFMA k-step),
-// LDS rows padded to 80 bytes so the 16 lanes of each quarter-wave hit 16
-// distinct 4-bank groups on their 16-byte fragment reads.
+// K slab 32 (one MFMA k-step), LDS rows padded to 80 bytes so the 16 lanes of each
+// quarter-wave hit 16 distinct 4-bank groups on their 16-byte fragment reads.
 // ---------------------------------------------------------------------------
 namespace nsmi {
 namespace {
@@ -619,21 +618,21 @@ struct BfArgs {
 
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 
-constexpr int kBfThreads = 512;
-
-template <int TERMS, typename TC, int ROLE>
-__global__ __launch_bounds__(kBfThreads) void k_gemm_bf16_nt(BfArgs g) {
-  constexpr int BM = 128, BN = 128, BK = 32, PITCH = BK + 8;  // in bf16 elements
+// TS x TS tiles: 128 with 8 waves (2 x 4, each 64 x 32), 64 with 4 (2 x 2, 32 x 32), 32 with 2
+// (1 x 2, 32 x 16); each thread stages one 16-byte chunk per plane and operand in all three
+template <int TS, int TERMS, typename TC, int ROLE>
+__global__ __launch_bounds__(TS * 4) void k_gemm_bf16_nt(BfArgs g) {
+  constexpr int BM = TS, BN = TS, BK = 32, PITCH = BK + 8;  // in bf16 elements
+  constexpr int WM = TS == 32 ? 1 : 2, WN = TS == 128 ? 4 : 2, WTM = BM / WM, WTN = BN / WN;
+  constexpr int FM = WTM / 16, FN = WTN / 16;
   constexpr int NP = (TERMS == 3) ? 2 : 1;                     // planes per operand
   __shared__ __attribute__((aligned(16))) uint16_t sA[2][NP][BM][PITCH];
   __shared__ __attribute__((aligned(16))) uint16_t sB[2][NP][BN][PITCH];
 
-  // 8 waves as 2 (m) x 4 (n), each wave a 64 x 32 block of the tile
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 2, wn = wave & 3;
-  const int nwg = g.tiles_m * g.tiles_n;
-  const int tile = xcd_remap(blockIdx.x, nwg);
-  const int tm = tile / g.tiles_n, tn = tile % g.tiles_n;
+  const int wm = wave / WN, wn = wave % WN;
+  int tm, tn;
+  tile_of(xcd_remap(blockIdx.x, g.tiles_m * g.tiles_n), g.tiles_m, g.tiles_n, tm, tn);
   const int64_t m0 = int64_t(tm) * BM, n0 = int64_t(tn) * BN;
 
   // each thread stages the 16-byte chunk tid % 4 of row tid / 4 of every tile plane
@@ -662,34 +661,34 @@ __global__ __launch_bounds__(kBfThreads) void k_gemm_bf16_nt(BfArgs g) {
     }
   };
 
-  f4 acc[4][2];
+  f4 acc[FM][FN];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f4{0, 0, 0, 0};
+    for (int j = 0; j < FN; ++j) acc[i][j] = f4{0, 0, 0, 0};
 
   // two fragment sets in registers: the MFMAs of K-step kt use set kt & 1 while
   // the fragments of step kt + 1 are read from the other LDS buffer
   const int fr = lane & 15, fk = (lane >> 4) * 8;
-  bf8 fa[2][NP][4], fb[2][NP][2];
+  bf8 fa[2][NP][FM], fb[2][NP][FN];
   auto frag = [&](auto set_c, int buf) {
     constexpr int S = decltype(set_c)::value;
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        fa[S][p][i] = *reinterpret_cast<const bf8*>(&sA[buf][p][wm * 64 + i * 16 + fr][fk]);
+      for (int i = 0; i < FM; ++i)
+        fa[S][p][i] = *reinterpret_cast<const bf8*>(&sA[buf][p][wm * WTM + i * 16 + fr][fk]);
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-        fb[S][p][j] = *reinterpret_cast<const bf8*>(&sB[buf][p][wn * 32 + j * 16 + fr][fk]);
+      for (int j = 0; j < FN; ++j)
+        fb[S][p][j] = *reinterpret_cast<const bf8*>(&sB[buf][p][wn * WTN + j * 16 + fr][fk]);
     }
   };
   auto mma = [&](auto set_c) {
     constexpr int S = decltype(set_c)::value;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < FN; ++j) {
         if constexpr (TERMS == 3) {
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[S][1][i], fb[S][0][j], acc[i][j], 0, 0, 0);
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[S][0][i], fb[S][1][j], acc[i][j], 0, 0, 0);
@@ -732,24 +731,45 @@ __global__ __launch_bounds__(kBfThreads) void k_gemm_bf16_nt(BfArgs g) {
   TC* C = static_cast<TC*>(g.C);
   const int kl = lane >> 4;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int64_t gm = m0 + wm * 64 + i * 16 + 4 * kl + r;  // bf16 16x16x32: rows 4*(l/16)+r
-        const int64_t gn = n0 + wn * 32 + j * 16 + fr;
+        const int64_t gm = m0 + wm * WTM + i * 16 + 4 * kl + r;  // bf16 16x16x32: rows 4*(l/16)+r
+        const int64_t gn = n0 + wn * WTN + j * 16 + fr;
         if (gm < g.M && gn < g.N) C[gm * g.ldc + gn] = TC(acc[i][j][r]);
       }
 }
 
-template <int TERMS, typename TC>
-void bf16_role(nsmi_ctx* ctx, int role, dim3 grid, const BfArgs& a) {
+template <int TS, int TERMS, typename TC>
+void bf16_role(nsmi_ctx* ctx, int role, BfArgs& a) {
+  a.tiles_m = int((a.M + TS - 1) / TS);
+  a.tiles_n = int((a.N + TS - 1) / TS);
+  const dim3 grid(unsigned(a.tiles_m) * unsigned(a.tiles_n)), block(TS * 4);
   switch (role) {
-    case kRoleHeff1: NSMI_LAUNCH_TIMED(ctx, (k_gemm_bf16_nt<TERMS, TC, kRoleHeff1>), grid, dim3(kBfThreads), a); break;
-    case kRoleHeff2: NSMI_LAUNCH_TIMED(ctx, (k_gemm_bf16_nt<TERMS, TC, kRoleHeff2>), grid, dim3(kBfThreads), a); break;
-    default: NSMI_LAUNCH_TIMED(ctx, (k_gemm_bf16_nt<TERMS, TC, kRoleEnv>), grid, dim3(kBfThreads), a); break;
+    case kRoleHeff1: NSMI_LAUNCH_TIMED(ctx, (k_gemm_bf16_nt<TS, TERMS, TC, kRoleHeff1>), grid, block, a); break;
+    case kRoleHeff2: NSMI_LAUNCH_TIMED(ctx, (k_gemm_bf16_nt<TS, TERMS, TC, kRoleHeff2>), grid, block, a); break;
+    default: NSMI_LAUNCH_TIMED(ctx, (k_gemm_bf16_nt<TS, TERMS, TC, kRoleEnv>), grid, block, a); break;
   }
+}
+
+// 128 x 128 (one workgroup per CU) where its rounds over the CUs are full enough: the three-term
+// product from 65% (3200 x 800 x 4000, 175 tiles: 106 us, 64 x 64 113; 3500 x 2800 x 700, 616: 65 / 71;
+// but 2560 x 2048 x 512, 320: 34 / 29; 2800 x 700 x 3500, 132: 95 / 71), the single-term one from 75%
+// (3000 x 2400 x 600, 456: 20 / 26; 3200 x 800 x 4000: 68 / 57).  Below it 64 x 64 while it has a tile
+// per CU (2400 x 600 x 3000, 380 tiles: 59 us, 32 x 32 72; 2048 x 512 x 2560, 256: 40 / 43), else
+// 32 x 32 (1556 x 421 x 2105, 175 tiles: 29 us, 64 x 64 34, 128 x 128 59; 800 x 200 x 1000: 10 / 14 / 28).
+template <int TERMS, typename TC>
+void bf16_tile(nsmi_ctx* ctx, int role, BfArgs& a) {
+  const int64_t big = ((a.M + 127) / 128) * ((a.N + 127) / 128);
+  const bool mid = ((a.M + 63) / 64) * ((a.N + 63) / 64) >= 256;
+  if (100 * big >= (TERMS == 3 ? 65 : 75) * 256 * ((big + 255) / 256))
+    bf16_role<128, TERMS, TC>(ctx, role, a);
+  else if (mid)
+    bf16_role<64, TERMS, TC>(ctx, role, a);
+  else
+    bf16_role<32, TERMS, TC>(ctx, role, a);
 }
 
 }  // namespace
@@ -761,14 +781,13 @@ void gemm_bf16_nt(nsmi_ctx* ctx, int64_t M, int64_t N, int64_t Kp, const uint16_
           "gemm_bf16: K must be positive and padded to 32, rows 16-byte aligned");
   require(terms == 1 || terms == 3, "gemm_bf16: terms must be 1 or 3");
   if (M == 0 || N == 0) return;
-  BfArgs a{Ahi, Alo, Bhi, Blo, C, M, N, Kp, lda, ldb, ldc, int((M + 127) / 128), int((N + 127) / 128)};
-  dim3 grid(unsigned(a.tiles_m) * unsigned(a.tiles_n));
+  BfArgs a{Ahi, Alo, Bhi, Blo, C, M, N, Kp, lda, ldb, ldc, 0, 0};
   if (terms == 3) {
-    if (c_double) bf16_role<3, double>(ctx, role, grid, a);
-    else bf16_role<3, float>(ctx, role, grid, a);
+    if (c_double) bf16_tile<3, double>(ctx, role, a);
+    else bf16_tile<3, float>(ctx, role, a);
   } else {
-    if (c_double) bf16_role<1, double>(ctx, role, grid, a);
-    else bf16_role<1, float>(ctx, role, grid, a);
+    if (c_double) bf16_tile<1, double>(ctx, role, a);
+    else bf16_tile<1, float>(ctx, role, a);
   }
   NSMI_LAUNCH_CHECK();
 }

@@ -45,6 +45,23 @@ def test_products_at_tile_edges(ctx, cl, cr, precision, u):
     assert np.linalg.norm(got - want) <= 8 * np.sqrt(K) * u * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("precision,bar", [("bf16x3", 2.0**-15), ("bf16", 2.0**-7)])
+@pytest.mark.parametrize("cl,cr", [(1, 1), (7, 9), (15, 17), (33, 31), (63, 65), (129, 95), (251, 259), (421, 449)])
+def test_bf16_products_at_tile_edges(ctx, cl, cr, precision, bar):
+    """Tiles of 32, 64 (1255 x 1036, 340 of them) and 128 (2105 x 1796).  Two products follow
+    each other, each with two operands rounded to 2^-9 (split in two: 2^-17, and 2^-18 for the
+    product of the low parts that is left out): at most 4 x 2^-9 and 5 x 2^-17 of the norm."""
+    import networksolvers_amd as ns
+    from oracle import chain
+    rng = np.random.default_rng(cl * 1000 + cr)
+    L, R = rng.standard_normal((cl, DW, cl)), rng.standard_normal((cr, DW, cr))
+    W = rng.standard_normal((DW, DW, D, D))
+    x = rng.standard_normal((cl, D, D, cr))
+    want = chain.heff2_apply(L, W, W, R, x)
+    got = ns.HeffMap(ctx.upload(L), ctx.upload(W), ctx.upload(W), ctx.upload(R), precision)(ctx.upload(x)).numpy()
+    assert np.linalg.norm(got - want) <= bar * np.linalg.norm(want)
+
+
 def _crand(rng, shape):
     return rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
 
