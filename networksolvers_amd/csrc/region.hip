@@ -209,13 +209,23 @@ __global__ void k_split_transpose(const double* __restrict__ X, int64_t rows, in
 }
 
 // H_eff mixing written as GEMM2's bf16 operand:
-// Y[(o*S + p/D2), (p%D2)*I + i] = sum_q Mx[p][q] X[o][q][i],  S = P / D2
+// Y[(o*S + p/D2), (p%D2)*I + i] = sum_q Mx[p][q] X[o][q][i],  S = P / D2,
+// for the PC outputs p of blockIdx.z (a multiple of 4).  Mx is padded with zeros to QMAX columns
+// and four rows in LDS, so the sums have no branches, four of them run side by side and
+// their coefficients come as 16-byte broadcasts: with a test of q < Q at every term and one
+// sum at a time the kernel waited for each LDS read (613 x 487, d = 2: 31 -> 16 us, 48 MB; the
+// whole apply at 400 x 300, d = 3: 273 -> 108 us, at 8 x 8: 29 -> 11). Two columns per thread, to
+// share those reads, gained nothing.
 template <int QMAX>
 __global__ __launch_bounds__(256) void k_mix_bf16_rows(const float* __restrict__ X, uint16_t* __restrict__ Yhi,
                                                        uint16_t* __restrict__ Ylo, const double* __restrict__ Mx,
-                                                       int64_t O, int P, int Q, int64_t I, int D2, int64_t Kp) {
-  __shared__ float sM[64 * 64];
-  for (int t = threadIdx.x; t < P * Q; t += blockDim.x) sM[t] = float(Mx[t]);
+                                                       int64_t O, int P, int Q, int64_t I, int D2, int64_t Kp, int PC) {
+  __shared__ __align__(16) float sM[64 * QMAX];
+  const int pb = blockIdx.z * PC, pe = min(pb + PC, P), PR = (pe - pb + 3) & ~3;
+  for (int t = threadIdx.x; t < PR * QMAX; t += 256) {
+    const int p = pb + t / QMAX, q = t % QMAX;
+    sM[t] = p < pe && q < Q ? float(Mx[p * Q + q]) : 0.f;
+  }
   __syncthreads();
   const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
   if (i >= I) return;
@@ -225,16 +235,21 @@ __global__ __launch_bounds__(256) void k_mix_bf16_rows(const float* __restrict__
     float x[QMAX];
 #pragma unroll
     for (int q = 0; q < QMAX; ++q) x[q] = (q < Q) ? xo[int64_t(q) * I] : 0.f;
-    for (int p = 0; p < P; ++p) {
-      const float* m = sM + p * Q;
-      float acc = 0.f;
+    for (int p = pb; p < pe; p += 4) {
+      const float* m = sM + (p - pb) * QMAX;
+      float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int q = 0; q < QMAX; ++q)
-        if (q < Q) acc += m[q] * x[q];
-      const int64_t idx = (o * S + p / D2) * Kp + int64_t(p % D2) * I + i;
-      const uint16_t h = bf16_rne(acc);
-      Yhi[idx] = h;
-      if (Ylo) Ylo[idx] = bf16_rne(acc - bf16_f32(h));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] += m[j * QMAX + q] * x[q];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (p + j < pe) {
+          const int64_t idx = (o * S + (p + j) / D2) * Kp + int64_t((p + j) % D2) * I + i;
+          const uint16_t h = bf16_rne(acc[j]);
+          Yhi[idx] = h;
+          if (Ylo) Ylo[idx] = bf16_rne(acc[j] - bf16_f32(h));
+        }
     }
   }
 }
@@ -274,13 +289,21 @@ void mix_f32_to_bf16_rows(nsmi_ctx* ctx, const float* X, uint16_t* Yhi, uint16_t
   require(P >= 1 && Q >= 1 && P <= 64 && Q <= 64 && D2 >= 1 && P % D2 == 0, "mix_bf16: bad P, Q, D2");
   if (O == 0 || I == 0) return;
   ProfScope ps(ctx, cls, 2.0 * double(O) * double(I) * P * Q, double(O) * double(I) * (P * 4.0 + Q * 4.0));
-  dim3 grid(unsigned((I + 255) / 256), unsigned(std::min<int64_t>(O, 65535)));
-  if (Q <= 16)
-    hipLaunchKernelGGL((k_mix_bf16_rows<16>), grid, dim3(256), 0, ctx->stream, X, Yhi, Ylo, Mx, O, P, Q, I, D2, Kp);
-  else if (Q <= 32)
-    hipLaunchKernelGGL((k_mix_bf16_rows<32>), grid, dim3(256), 0, ctx->stream, X, Yhi, Ylo, Mx, O, P, Q, I, D2, Kp);
-  else
-    hipLaunchKernelGGL((k_mix_bf16_rows<64>), grid, dim3(256), 0, ctx->stream, X, Yhi, Ylo, Mx, O, P, Q, I, D2, Kp);
+  // the outputs split into chunks of 4 k until the grid holds about 2048 waves
+  const int64_t oy = std::min<int64_t>(O, 65535), ix = (I + 255) / 256, waves = 4 * ix * oy;
+  const int64_t want = std::max<int64_t>(1, (2048 + waves - 1) / waves);
+  const int quads = (P + 3) / 4, split = int(std::min<int64_t>(quads, want));
+  const int PC = 4 * ((quads + split - 1) / split);
+  const dim3 grid{unsigned(ix), unsigned(oy), unsigned((P + PC - 1) / PC)};
+#define NSMI_MIX_GO(QMAX)                                                                                          \
+  hipLaunchKernelGGL((k_mix_bf16_rows<QMAX>), grid, dim3(256), 0, ctx->stream, X, Yhi, Ylo, Mx, O, P, Q, I, D2, Kp, \
+                     PC)
+  if (Q <= 12) NSMI_MIX_GO(12);
+  else if (Q <= 20) NSMI_MIX_GO(20);
+  else if (Q <= 32) NSMI_MIX_GO(32);
+  else if (Q <= 48) NSMI_MIX_GO(48);
+  else NSMI_MIX_GO(64);
+#undef NSMI_MIX_GO
   NSMI_LAUNCH_CHECK();
 }
 

@@ -62,6 +62,21 @@ def test_bf16_products_at_tile_edges(ctx, cl, cr, precision, bar):
     assert np.linalg.norm(got - want) <= bar * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("Dw,d,sites", [(1, 2, 1), (6, 2, 1), (7, 2, 1), (5, 2, 2), (3, 3, 2), (5, 3, 2), (7, 3, 2)])
+@pytest.mark.parametrize("cl,cr", [(2, 255), (300, 257)])
+def test_bf16_mixing_widths(ctx, Dw, d, sites, cl, cr):
+    """Widths (Dw d^sites = 2 to 63) on both sides of the padded ones (12, 20, 32, 48, 64), with an
+    output count that is no multiple of four, columns at the edge of a workgroup, few and many rows."""
+    import networksolvers_amd as ns
+    from oracle import chain
+    rng = np.random.default_rng(Dw * 100 + d)
+    L, R, W = rng.standard_normal((cl, Dw, cl)), rng.standard_normal((cr, Dw, cr)), rng.standard_normal((Dw, Dw, d, d))
+    x = rng.standard_normal((cl,) + (d,) * sites + (cr,))
+    want = chain.heff2_apply(L, W, W, R, x) if sites == 2 else chain.heff1_apply(L, W, R, x)
+    H = ns.HeffMap(ctx.upload(L), ctx.upload(W), ctx.upload(W) if sites == 2 else None, ctx.upload(R), "bf16x3")
+    assert np.linalg.norm(H(ctx.upload(x)).numpy() - want) <= 2.0**-15 * np.linalg.norm(want)
+
+
 def _crand(rng, shape):
     return rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
 
