@@ -62,12 +62,16 @@ inline BidiagExchange bidiag_exchange(int cl, int gmax, int groups, bool all) {
   return x;
 }
 
+// waves per SIMD: eight-wave workgroups of a one-XCD group keep to 128 VGPRs, so that two fit
+// a CU
+constexpr int bidiag_occupancy(int nw, BidiagMode mode) {
+  return nw == 8 && (mode == kOneXcd || mode == kOneXcdSliced) ? 4 : 1;
+}
+
 template <int CL, int RW, int NW, BidiagMode MODE, int GMAX = 16>
-// eight-wave workgroups of a one-XCD group keep to 128 VGPRs, so that two fit a CU
-__global__ __launch_bounds__(64 * NW, NW == 8 && (MODE == kOneXcd || MODE == kOneXcdSliced) ? 4 : 1) void k_bidiag(double* __restrict__ X, int r, int s, double* __restrict__ d,
-                                                    double* __restrict__ e, double* __restrict__ tauL,
-                                                    double* __restrict__ tauR, double* __restrict__ xch,
-                                                    unsigned* __restrict__ ctl, int groups, int want) {
+__global__ __launch_bounds__(64 * NW, bidiag_occupancy(NW, MODE)) void k_bidiag(
+    double* __restrict__ X, int r, int s, double* __restrict__ d, double* __restrict__ e, double* __restrict__ tauL,
+    double* __restrict__ tauR, double* __restrict__ xch, unsigned* __restrict__ ctl, int groups, int want) {
   constexpr int STEP = CL > 16 ? 4 : (CL > 8 ? 2 : 1);
   constexpr int NP = 64 * (CL + STEP - 1), NT = 64 * NW, NY = (64 * CL + NT - 1) / NT;
   __shared__ double comb[NW][NP];    // from the current block on

@@ -530,13 +530,14 @@ bool tiles_fill(const GemmDesc& d) {
 // else the 32 x 32 tile, whose deep slabs and many workgroups hide the latency: in FP64 it
 // is never behind 64 x 64 by more than the runs differ (1024 x 1024 x 1024: 44 us against
 // 50-55; 1536 x 1536 x 1024: 93 against 115-138), which is therefore not built for FP64.
-// Up to 64 tiles of 32 x 32 the wave form, while K is short enough for its uncoalesced reads (512
-// in FP64, 1024 in FP32); us, wave form / 32 x 32 with its split: FP64 60, 60, 60: 3.5 / 4.4;
-// 394, 64, 394: 5.5-6.1 / 8.2; 400, 100, 500: 6.5 / 8.7; FP32 64, 64, 1024: 5.4-7.0 / 7.9; 400, 100,
-// 500: 4.4 / 7.6.  It loses at more tiles (FP64 320, 256, 64, 80 tiles: 5.2 / 4.1; 384, 384, 384: 11-18
-// / 8.7) and longer K (FP64 64, 64, 1024: 7.4-11.9 / 9.0; 64, 200, 2048: 11-19 / 10.8).  In
-// FP32 64 x 64 wins from about two full rounds (1536 x 1280 x 1024: 40 us against 45;
+// In FP32 64 x 64 wins from about two full rounds (1536 x 1280 x 1024: 40 us against 45;
 // 2176 x 2176 x 1024: 94 against 108) and loses before (1024 x 1024 x 1024: 26 against 24).
+// Up to 64 tiles of 32 x 32 the wave form, while K is short enough for its uncoalesced reads
+// (512 in FP64, 1024 in FP32); us, wave form / 32 x 32 with its split: FP64 60, 60, 60: 3.5 /
+// 4.4; 394, 64, 394: 5.5-6.1 / 8.2; 400, 100, 500: 6.5 / 8.7; FP32 64, 64, 1024: 5.4-7.0 / 7.9;
+// 400, 100, 500: 4.4 / 7.6.  It loses at more tiles (FP64 320, 256, 64, 80 tiles: 5.2 / 4.1;
+// 384, 384, 384: 11-18 / 8.7) and longer K (FP64 64, 64, 1024: 7.4-11.9 / 9.0; 64, 200, 2048:
+// 11-19 / 10.8).
 template <typename T, typename TBm, typename TCm, int ROLE>
 void launch_role(nsmi_ctx* ctx, const GemmDesc& d, GemmArgs<T, TBm, TCm>& a) {
   if (((d.M + 31) / 32) * ((d.N + 31) / 32) * d.batch <= 64 && d.K <= 4096 / int64_t(sizeof(T)))

@@ -421,11 +421,11 @@ void small_sym_eigh(int n, const double* A, double* w, double* V);  // host Jaco
 
 // ---- tridiagonal reduction (eig.hip) ----------------------------------------
 // Householder reduction of a symmetric n x n device matrix to tridiagonal form in
-// LAPACK's dsytrd "lower" layout (one cooperative launch); false when n is outside
+// LAPACK's dsytrd "lower" order, reflectors in place (one launch); false when n is outside
 // [2, kSytrdMax] or the device cannot co-schedule the grid.
 constexpr int kSytrdMax = 1024;
 // one asynchronous tridiagonal reduction: its exchange and flag buffers, and the
-// host copy of the two failure flags (barrier time-out, non-finite d or e)
+// host copy of the two failure flags (an exchange that timed out, non-finite d or e)
 struct SytrdRun {
   std::unique_ptr<Scratch> xch, flags;
   unsigned* host_flags = nullptr;  // two flags in pinned stage memory
@@ -450,7 +450,7 @@ void apply_reflectors(nsmi_ctx* ctx, const double* Vt, const double* tau, int m,
 
 // ---- own dense SVD / tridiagonal eigensolver pieces (svd.hip) -------------------
 // One-launch Householder bidiagonalisation of a tall r x s device matrix X (r >= s,
-// row-major; reflectors left in place, see svd.hip), d (s), e, tauR (s - 1), tauL (s).
+// row-major; reflectors left in place, see bidiag.h), d (s), e, tauR (s - 1), tauL (s).
 // Enqueues the launch and the copy of its two failure flags (as sytrd_launch); false
 // with nothing launched when the size is outside the kernels' range or the grid cannot
 // be co-scheduled.
