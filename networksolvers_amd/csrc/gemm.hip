@@ -426,14 +426,16 @@ __global__ __launch_bounds__(512) void k_gemm_wave(GemmArgs<T, TBm, TCm> g) {
   for (int r = 0; r < 4; ++r) part[wave][r][lane] = acc[r];
   __syncthreads();
   if (tid >= 256) return;
-  T sum = T(0);  // waves 0..3 write item r = wave of every lane
+  // waves 0..3 write item r = wave of every lane; as in k_splitk_reduce the partial sums of
+  // a split K are added and scaled in FP64 and rounded once, to C's type
+  double sum = 0.0;
 #pragma unroll
-  for (int w = 0; w < NW; ++w) sum += part[w][wave][lane];
+  for (int w = 0; w < NW; ++w) sum += double(part[w][wave][lane]);
   const int64_t gm = m0 + out_row<T>(kl, wave), gn = n0 + ml;
   if (gm >= g.M || gn >= g.N) return;
   TCm* const C = g.C + bz * g.sC;
-  T v = g.alpha * sum;
-  if (g.beta != T(0)) v += g.beta * T(C[gm * g.ldc + gn]);
+  double v = double(g.alpha) * sum;
+  if (g.beta != T(0)) v += double(g.beta) * double(C[gm * g.ldc + gn]);
   C[gm * g.ldc + gn] = TCm(v);
 }
 

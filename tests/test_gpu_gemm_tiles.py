@@ -122,3 +122,20 @@ def test_environment_products_at_tile_edges(ctx, ca, cb, side):
     got = ns.env_update(ctx.upload(E), ctx.upload(A), ctx.upload(W), side).numpy()
     K = DW * max(ca, cb)
     assert np.linalg.norm(got - want) <= 8 * np.sqrt(K) * 2.0**-53 * np.linalg.norm(want)
+
+
+def test_fp32_partial_sums_are_added_in_fp64(ctx):
+    """The FP32 form writes y in FP64: where a product splits its K = 512 over waves or
+    workgroups, the partial sums are added in FP64 and not rounded on the way.  Two terms,
+    2^24 at k = 0 and 1 at k = 144, lie in different parts of every split (parts of 16 dealt to
+    8 waves; parts of 128): their sum needs 25 bits and comes out exactly."""
+    import networksolvers_amd as ns
+    n = 512
+    L, W, R = np.ones((1, 1, 1)), np.eye(D).reshape(1, 1, D, D), np.zeros((n, 1, n))
+    R[0, 0, :] = 1.0
+    x = np.zeros((1, D, D, n))
+    x[0, 0, 0, 0], x[0, 0, 0, 144] = 2.0**24, 1.0
+    H = ns.HeffMap(ctx.upload(L), ctx.upload(W), ctx.upload(W), ctx.upload(R), "fp32")
+    got = H(ctx.upload(x)).numpy()
+    assert got[0, 0, 0, 0] == 2.0**24 + 1.0
+    assert np.count_nonzero(got) == 1
