@@ -16,10 +16,11 @@
 // step and to hear, for that word, from everyone who reads what it empties.
 //
 // The workgroups that exchange most are placed on one XCD where they fit, so that the
-// words stay in that XCD's L2: they are written by plain stores (which stop in the L2
-// that the group shares) and read by relaxed agent-scope loads (never from the CU's own
-// cache; 0.16 us inside an XCD, 0.3 us across).  Words that cross XCDs are written by
-// relaxed agent-scope stores, which leave nothing in the writer's L2.
+// words stay in that XCD's L2: they are written by relaxed atomic stores of workgroup scope
+// (never by plain ones, which the compiler may split, merge or move; they stop in the L2
+// that the group shares, as every store that leaves a CU does) and read by relaxed agent-scope
+// loads (never from the CU's own cache; 0.16 us inside an XCD, 0.3 us across).  Words that
+// cross XCDs are written by relaxed agent-scope stores, which leave nothing in the writer's L2.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -63,10 +64,10 @@ __device__ inline void st_agent(T* p, T v) {
 __device__ inline unsigned add_agent(unsigned* p) {
   return __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// a word for readers inside the group: plain when the group shares an L2
+// a word for readers inside the group; local: the group shares an L2
 __device__ inline void st_group(double* p, double v, bool local) {
   if (local)
-    *p = v;
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   else
     st_agent(p, v);
 }
