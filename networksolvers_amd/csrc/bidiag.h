@@ -299,13 +299,16 @@ __global__ __launch_bounds__(64 * NW, bidiag_occupancy(NW, MODE)) void k_bidiag(
 #pragma unroll
           for (int sl = 0; sl < RW; ++sl) xn[sl] = lane_bcast(row[sl][0], min(jl + 1, 63));
           if (at0) y2[0] = 0.0;
-        } else if (q == 1) {
-          if (jl == 63) {
-            alpha2 = lane_bcast(y2[1], 0);
+        }
+        if constexpr (CA > 1) {
+          if (q == 1) {
+            if (jl == 63) {
+              alpha2 = lane_bcast(y2[1], 0);
 #pragma unroll
-            for (int sl = 0; sl < RW; ++sl) xn[sl] = lane_bcast(row[sl][1], 0);
+              for (int sl = 0; sl < RW; ++sl) xn[sl] = lane_bcast(row[sl][1], 0);
+            }
+            if (at1) y2[1] = 0.0;
           }
-          if (at1) y2[1] = 0.0;
         }
         red[RW] = fma(y2[q], y2[q], red[RW]);
 #pragma unroll
@@ -334,9 +337,12 @@ __global__ __launch_bounds__(64 * NW, bidiag_occupancy(NW, MODE)) void k_bidiag(
         if (q == 0) {
 #pragma unroll
           for (int sl = 0; sl < RW; ++sl) row[sl][0] = at0 ? xn[sl] : (lane == jl ? un[sl] : row[sl][0]);
-        } else if (q == 1) {
+        }
+        if constexpr (CA > 1) {
+          if (q == 1) {
 #pragma unroll
-          for (int sl = 0; sl < RW; ++sl) row[sl][1] = at1 ? xn[sl] : row[sl][1];
+            for (int sl = 0; sl < RW; ++sl) row[sl][1] = at1 ? xn[sl] : row[sl][1];
+          }
         }
       }
       // row j is finished: its owner stores d_j, e_j and v_j (u's of earlier blocks are stored)
@@ -345,8 +351,8 @@ __global__ __launch_bounds__(64 * NW, bidiag_occupancy(NW, MODE)) void k_bidiag(
         if (rid[sl] == j) {
           double* const xr = X + size_t(j) * s + cb;
 #pragma unroll
-          for (int q = 0; q < CL; ++q) {
-              const int c = lane + 64 * q;
+          for (int q = 0; q < CA; ++q) {  // the columns left: cb + 64 CA >= s
+            const int c = lane + 64 * q;
             double v = y2[q] * scal2;
             if (q == 0) v = lane < jl ? row[sl][0] : (lane == jl ? beta : (at0 ? beta2 : v));
             if (q == 1 && at1) v = beta2;
