@@ -131,6 +131,11 @@ int nsmi_pool_trim(nsmi_ctx* ctx);
    barrier and the call reports NSMI_ERR_SOLVER, exactly as when a barrier wait
    gives up; the context stays usable. */
 int nsmi_inject_barrier_timeout(nsmi_ctx* ctx, int count);
+/* The same for their placement: the next `count` of them do not get the XCDs that they ask
+   for.  A group on one XCD then leaves without having started and is launched again over
+   the whole device; a group over all XCDs is formed in the grid's order.  Results are
+   those of the usual placement, bit for bit. */
+int nsmi_inject_misplacement(nsmi_ctx* ctx, int count);
 
 /* ---------------------------------------------------------------- tensors */
 int nsmi_tensor_create(nsmi_ctx* ctx, int dtype, int rank, const int64_t* dims, nsmi_tensor** out);

@@ -70,6 +70,7 @@ SIGNATURES = {
     "nsmi_pool_stats": (C.c_int, [_VP, C.POINTER(C.c_size_t), C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]),
     "nsmi_pool_trim": (C.c_int, [_VP]),
     "nsmi_inject_barrier_timeout": (C.c_int, [_VP, C.c_int]),
+    "nsmi_inject_misplacement": (C.c_int, [_VP, C.c_int]),
     "nsmi_heff_apply_noalloc": (C.c_int, [_VP, _VP, _VP, _VP]),
     "nsmi_noalloc_scratch_bytes": (C.c_size_t, []),
     "nsmi_tensor_create": (C.c_int, [_VP, C.c_int, C.c_int, _I64P, _PP]),

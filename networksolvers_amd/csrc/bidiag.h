@@ -26,7 +26,7 @@
 // Exchange (group.h: words are polled until they are there), thread t handling the
 // columns c = t mod NT, by MODE:
 //   kOneGroup  one workgroup, through LDS;
-//   kOneXcd    G workgroups on one XCD: each publishes its S, everyone adds the G values
+//   kOneXcd    G workgroups on XCD `want` (want < 0: anywhere): each publishes its S, everyone adds the G values
 //              of every column in order;
 //   kAllXcds   8 GW workgroups, GW on each XCD: each publishes its S to its XCD; workgroup w
 //              of each XCD adds its slice of the columns over that XCD's GW workgroups;
@@ -62,10 +62,10 @@ inline BidiagExchange bidiag_exchange(int cl, int gmax, int groups, bool all) {
   return x;
 }
 
-// waves per SIMD: eight-wave workgroups of a one-XCD group keep to 128 VGPRs, so that two fit
-// a CU
+// waves per SIMD: the workgroups of a one-XCD group keep to half of a CU's registers, so that
+// two fit a CU
 constexpr int bidiag_occupancy(int nw, BidiagMode mode) {
-  return nw == 8 && (mode == kOneXcd || mode == kOneXcdSliced) ? 4 : 1;
+  return mode == kOneXcd || mode == kOneXcdSliced ? nw / 2 : 1;
 }
 
 template <int CL, int RW, int NW, BidiagMode MODE, int GMAX = 16>
@@ -80,6 +80,9 @@ __global__ __launch_bounds__(64 * NW, bidiag_occupancy(NW, MODE)) void k_bidiag(
   __shared__ double part[MODE == kAllXcds || MODE == kOneXcdSliced ? NW : 1][64];
   __shared__ double s_alpha, s_sig;
   __shared__ int s_ok, s_place;
+  // beside one workgroup of another group, wherever that one lies in a CU's 160 KB
+  static_assert(MODE == kAllXcds || sizeof(comb) + sizeof(yrow) + sizeof(ys) + sizeof(zs) + sizeof(part) < 160 * 1024 / 3,
+                "two workgroups of one-XCD groups share a CU");
   // the wave's index and the workgroup's place are wave-uniform: branches on them are scalar
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   unsigned* const fail = ctl + kCtlFail;
@@ -89,10 +92,11 @@ __global__ __launch_bounds__(64 * NW, bidiag_occupancy(NW, MODE)) void k_bidiag(
   constexpr bool ALL = MODE == kAllXcds, SLICED = ALL || MODE == kOneXcdSliced;
   if (MODE == kOneXcd || MODE == kOneXcdSliced) {
     G = groups;
-    g = place_one_xcd(ctl, G, want, &local, &s_place);
+    local = want >= 0;
+    g = local ? place_one_xcd(ctl, G, want, &s_place) : place_spread(ctl, &s_place);
     if (g < 0) return;
   } else if (MODE == kAllXcds) {
-    if (!place_all_xcds(ctl, GW, &xx, &ww, &local, &s_place)) return;
+    if (!place_all_xcds(ctl, GW, want, &xx, &ww, &local, &s_place)) return;
     G = kXcds * GW;
     g = ww * kXcds + xx;
   }

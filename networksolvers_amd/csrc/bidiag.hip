@@ -10,15 +10,17 @@
 namespace nsmi {
 namespace {
 
-// Two groups at a time may hold an XCD (their workgroups fit two to a CU), and a group
-// that is only partly resident waits for the rest of itself, so no third one may start
-// there.  Each stream that launches such groups is given one of the 16 places (8 XCDs
-// x 2) for its life, spread over the XCDs first.  With more than 16 streams a place is
-// shared: a launch then waits for what the others sharing it have queued (an event per
+// Two groups at a time may hold an XCD (kGroupsPerXcd: their workgroups, at most one for
+// each of its CUs, fit two to a CU, and nothing but their members stays on the device, see
+// place_one_xcd), so both become resident; with a third one each could have a part of its
+// CUs and none enough.  Each stream that launches such groups is given one of the 16 places
+// (8 XCDs x 2) for its life, spread over the XCDs first.  With more than 16 streams a place
+// is shared: a launch then waits for what the others sharing it have queued (an event per
 // stream, under the lock, so that two of them cannot pass each other).
+constexpr int kCusPerXcd = 32, kGroupsPerXcd = 2;
 struct XcdPlaces {
   std::mutex mu;
-  std::vector<hipStream_t> users[2 * kXcds];
+  std::vector<hipStream_t> users[kGroupsPerXcd * kXcds];
   hipEvent_t ev = nullptr;
 };
 XcdPlaces& places_of(int device) {
@@ -34,7 +36,7 @@ void launch_on_one_xcd(nsmi_ctx* ctx, const std::function<void(int)>& launch) {
   XcdPlaces& p = places_of(ctx->device);
   std::lock_guard<std::mutex> lock(p.mu);
   int at = -1, best = 0;
-  for (int i = 0; i < 2 * kXcds; ++i) {
+  for (int i = 0; i < kGroupsPerXcd * kXcds; ++i) {
     for (hipStream_t s : p.users[i])
       if (s == ctx->stream) at = i;
     if (p.users[i].size() < p.users[best].size()) best = i;
@@ -64,6 +66,38 @@ unsigned reduction_fail0(nsmi_ctx* ctx, int G) {
   return 1u;
 }
 
+bool take_misplacement(nsmi_ctx* ctx) {
+  if (ctx->inject_misplaced <= 0) return false;
+  --ctx->inject_misplaced;
+  return true;
+}
+
+bool one_xcd_groups(nsmi_ctx* ctx) {
+  int xcds = 0, ncu = 0;
+  NSMI_HIP(hipDeviceGetAttribute(&xcds, hipDeviceAttributeNumberOfXccs, ctx->device));
+  NSMI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
+  return xcds == kXcds && ncu >= kXcds * kCusPerXcd;
+}
+
+bool launch_cooperative(nsmi_ctx* ctx, const void* fn, int groups, int threads, void** args) {
+  int coop = 0, ncu = 0, per_cu = 0;
+  NSMI_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device));
+  NSMI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
+  NSMI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, 0));
+  if (!coop || per_cu < 1 || groups > ncu * per_cu) return false;
+  const hipError_t st = hipLaunchCooperativeKernel(fn, dim3(unsigned(groups)), dim3(unsigned(threads)), args, 0,
+                                                   ctx->stream);
+  if (st != hipSuccess) (void)hipGetLastError();
+  return st == hipSuccess;
+}
+
+void reduction_readback(nsmi_ctx* ctx, SytrdRun& run) {
+  run.host_flags = static_cast<unsigned*>(stage_take(ctx, kCtlHostWords * sizeof(unsigned)));
+  for (int i = 0; i < kCtlHostWords; ++i) run.host_flags[i] = 0u;
+  NSMI_HIP(hipMemcpyAsync(run.host_flags, run.flags->as<unsigned>() + kCtlFail, kCtlHostWords * sizeof(unsigned),
+                          hipMemcpyDeviceToHost, ctx->stream));
+}
+
 namespace {
 
 struct BidiagPlan {
@@ -74,6 +108,7 @@ struct BidiagPlan {
 };
 template <int CL, int RW, int NW, BidiagMode MODE, int GMAX>
 BidiagPlan plan_of() {
+  static_assert(MODE == kOneGroup || GMAX <= kCusPerXcd, "at most one workgroup for each CU of an XCD");
   return {reinterpret_cast<const void*>(k_bidiag<CL, RW, NW, MODE, GMAX>), MODE, CL, 64 * NW, GMAX, RW * NW};
 }
 
@@ -89,7 +124,8 @@ BidiagPlan plan_of() {
 //   all XCDs: 3.7 at 512 x 512, 4.2 at 700 x 700, 4.5 at 1000 x 1000 (5.2 on one XCD), 5.9 at
 //   2048 x 2048, 5.8 at 4000 x 1000.
 // One-XCD groups go out as ordinary launches (at most 32 workgroups, places_of); the
-// others need up to one workgroup on every CU and take the cooperative launch.
+// others need up to one workgroup on every CU and take the cooperative launch, and so does a
+// one-XCD group that was not placed or that the device has no XCDs for.
 BidiagPlan bidiag_plan(int r, int s) {
   if (s <= 64) {
     if (r <= 32) return plan_of<1, 4, 8, kOneGroup, 1>();
@@ -136,18 +172,11 @@ int bidiag_groups(int r, int s) {
 }
 
 bool bidiag_launch(nsmi_ctx* ctx, double* X, int r, int s, double* d, double* e, double* tauL, double* tauR,
-                   SytrdRun& run) {
+                   SytrdRun& run, bool spread) {
   const int G = bidiag_groups(r, s);
   if (G == 0) return false;
   const BidiagPlan p = bidiag_plan(r, s);
   int groups = plan_groups(p, r, s);
-  if (p.mode == kAllXcds) {
-    int coop = 0, ncu = 0, per_cu = 0;
-    NSMI_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device));
-    NSMI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
-    NSMI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, p.fn, p.threads, 0));
-    if (!coop || per_cu < 1 || G > ncu * per_cu) return false;
-  }
   BidiagExchange x{};
   if (p.mode != kOneGroup) x = bidiag_exchange(p.cl, p.gmax, groups, p.mode == kAllXcds);
   run.xch.reset(new Scratch(ctx, sizeof(double) * std::max<size_t>(x.words, 1)));
@@ -159,31 +188,25 @@ bool bidiag_launch(nsmi_ctx* ctx, double* X, int r, int s, double* d, double* e,
                      unsigned(3 * 64 * p.cl), unsigned(std::max(x.per, 1)), unsigned(x.used), ctl, int(kCtlWords),
                      reduction_fail0(ctx, G));
   NSMI_LAUNCH_CHECK();
-  int rr = r, ss = s, want = 0;
+  int rr = r, ss = s, want = -1;
   void* args[] = {&X, &rr, &ss, &d, &e, &tauL, &tauR, &xp, &ctl, &groups, &want};
   {
     // algorithmic work of a Householder bidiagonalisation: 4 s^2 (r - s / 3) flops
     ProfScope ps(ctx, NSMI_K_FACT_REDUCE, 4.0 * double(s) * s * (double(r) - double(s) / 3.0),
                  16.0 * double(r) * s);
-    if (p.mode == kAllXcds) {
-      const hipError_t st =
-          hipLaunchCooperativeKernel(p.fn, dim3(unsigned(G)), dim3(unsigned(p.threads)), args, 0, ctx->stream);
-      if (st != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-      }
-    } else if (p.mode == kOneGroup) {
+    if (p.mode == kOneGroup) {
       NSMI_HIP(hipLaunchKernel(p.fn, dim3(1), dim3(unsigned(p.threads)), args, 0, ctx->stream));
+    } else if (p.mode == kAllXcds || spread || !one_xcd_groups(ctx)) {
+      if (p.mode == kAllXcds && !take_misplacement(ctx)) want = 0;
+      if (!launch_cooperative(ctx, p.fn, G, p.threads, args)) return false;
     } else {
       launch_on_one_xcd(ctx, [&](int xcd) {
-        want = xcd;
+        want = take_misplacement(ctx) ? kXcds : xcd;  // kXcds: none has this number
         NSMI_HIP(hipLaunchKernel(p.fn, dim3(unsigned(kXcds * G)), dim3(unsigned(p.threads)), args, 0, ctx->stream));
       });
     }
   }
-  run.host_flags = static_cast<unsigned*>(stage_take(ctx, 2 * sizeof(unsigned)));
-  run.host_flags[0] = run.host_flags[1] = 0u;
-  NSMI_HIP(hipMemcpyAsync(run.host_flags, ctl + kCtlFail, 2 * sizeof(unsigned), hipMemcpyDeviceToHost, ctx->stream));
+  reduction_readback(ctx, run);
   return true;
 }
 

@@ -409,6 +409,13 @@ int nsmi_inject_barrier_timeout(nsmi_ctx* ctx, int count) {
   API_END(ctx)
 }
 
+int nsmi_inject_misplacement(nsmi_ctx* ctx, int count) {
+  if (!ctx || count < 0) return NSMI_ERR_INVALID;
+  API_BEGIN(ctx)
+  ctx->inject_misplaced = count;
+  API_END(ctx)
+}
+
 int nsmi_tensor_create(nsmi_ctx* ctx, int dtype, int rank, const int64_t* dims, nsmi_tensor** out) {
   if (!ctx || !out) return NSMI_ERR_INVALID;
   API_BEGIN(ctx)

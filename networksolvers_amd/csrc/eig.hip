@@ -289,27 +289,21 @@ void apply_q_lower(nsmi_ctx* ctx, const double* rho, const double* tau, int n, d
 // A: n x n symmetric on the device (row-major == column-major), overwritten with the
 // reflectors as k_sytrd leaves them (LAPACK's lower layout without d and e); d (n), e and
 // tau (n - 1) on the device.  sytrd_launch enqueues the reduction on ctx->stream and the
-// copy of its two failure flags into run.host_flags; it returns false, with nothing
+// copy of its control words into run.host_flags; it returns false, with nothing
 // launched, when n is outside the supported range or the device cannot co-schedule the
-// grid (the caller then uses the library path).  sytrd_check reads the flags once the
-// stream has passed the copy.
+// grid (the caller then uses the library path).  Once the stream has passed the copy,
+// reduction_unplaced tells whether the group never started (A is then as it was, and the
+// caller launches again, spread) and sytrd_check reads the flags.
 //
 // A group on one XCD goes out as an ordinary launch: a cooperative launch waits for the
 // whole device to drain, which would serialise the independent solves that share the
 // GPU; that the group becomes resident rests on its place on the XCD
-// (launch_on_one_xcd), and the bounded polls turn the pathological case into an error,
-// not a hang.  A spread group takes the cooperative launch and its co-residency check.
-bool sytrd_launch(nsmi_ctx* ctx, double* A, int n, double* d, double* e, double* tau, SytrdRun& run) {
+// (launch_on_one_xcd), and its placement ends in a bounded time (group.h).  A spread
+// group takes the cooperative launch and its co-residency check.
+bool sytrd_launch(nsmi_ctx* ctx, double* A, int n, double* d, double* e, double* tau, SytrdRun& run, bool spread) {
   if (n < 2 || n > kSytrdMax) return false;
   const TriPlan p = tri_plan(n);
   int G = (n + p.rows - 1) / p.rows;
-  if (p.spread) {
-    int coop = 0, ncu = 0, per_cu = 0;
-    NSMI_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device));
-    NSMI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
-    NSMI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, p.fn, p.threads, 0));
-    if (!coop || per_cu < 1 || G > ncu * per_cu) return false;
-  }
   const size_t words = 6 * 64 * size_t(p.cl);
   run.xch.reset(new Scratch(ctx, sizeof(double) * words));
   run.flags.reset(new Scratch(ctx, sizeof(unsigned) * kCtlWords));
@@ -322,28 +316,21 @@ bool sytrd_launch(nsmi_ctx* ctx, double* A, int n, double* d, double* e, double*
   void* args[] = {&A, &nn, &d, &e, &tau, &xp, &ctl, &G, &want};
   {
     ProfScope ps(ctx, NSMI_K_FACT_REDUCE, 4.0 / 3.0 * double(n) * n * n, 16.0 * double(n) * n);
-    if (p.spread) {
-      const hipError_t st =
-          hipLaunchCooperativeKernel(p.fn, dim3(unsigned(G)), dim3(unsigned(p.threads)), args, 0, ctx->stream);
-      if (st != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-      }
+    if (p.spread || spread || !one_xcd_groups(ctx)) {
+      if (!launch_cooperative(ctx, p.fn, G, p.threads, args)) return false;
     } else {
       launch_on_one_xcd(ctx, [&](int xcd) {
-        want = xcd;
+        want = take_misplacement(ctx) ? kXcds : xcd;  // kXcds: none has this number
         NSMI_HIP(hipLaunchKernel(p.fn, dim3(unsigned(kXcds * G)), dim3(unsigned(p.threads)), args, 0, ctx->stream));
       });
     }
   }
-  run.host_flags = static_cast<unsigned*>(stage_take(ctx, 2 * sizeof(unsigned)));
-  run.host_flags[0] = run.host_flags[1] = 0u;
-  NSMI_HIP(hipMemcpyAsync(run.host_flags, ctl + kCtlFail, 2 * sizeof(unsigned), hipMemcpyDeviceToHost, ctx->stream));
+  reduction_readback(ctx, run);
   return true;
 }
 
 void sytrd_check(const SytrdRun& run) {
-  if (run.host_flags[0])
+  if (run.host_flags[0] || reduction_unplaced(run))
     fail(NSMI_ERR_SOLVER, "sytrd: a workgroup of the tridiagonal reduction timed out at a grid barrier");
   // the tridiagonal solver is never handed NaN or Inf
   if (run.host_flags[1]) fail(NSMI_ERR_NOT_FINITE, "factorize: non-finite entries in the matrix to be factorized");

@@ -321,11 +321,20 @@ void fact_readback(nsmi_ctx* ctx, FactCore& f) {
   NSMI_HIP(hipMemcpyAsync(f.wh, f.w->p, sizeof(double) * f.iso, hipMemcpyDeviceToHost, ctx->stream));
 }
 
-// after the reduction's flags are on the host: every eigenvalue of T by bisection
-// (descending), copied to the host; the eigenvectors wait for the truncation
+void fact_syevd(nsmi_ctx* ctx, FactCore& f);
+
+// after the reduction's flags are on the host (a group that never started is launched again
+// first, spread): every eigenvalue of T by bisection (descending), copied to the host; the
+// eigenvectors wait for the truncation
 void fact_tri_solve(nsmi_ctx* ctx, FactCore& f) {
-  sytrd_check(f.sr);
   const int64_t iso = f.iso;
+  for (int i = 0; i < kRelaunches && reduction_unplaced(f.sr); ++i) {
+    f.tri = sytrd_launch(ctx, f.rho->as<double>(), int(iso), f.w->as<double>(), f.e->as<double>(),
+                         f.tau->as<double>(), f.sr, true);
+    if (!f.tri) return fact_syevd(ctx, f);
+    NSMI_HIP(hipStreamSynchronize(ctx->stream));
+  }
+  sytrd_check(f.sr);
   f.lam.reset(new Scratch(ctx, sizeof(double) * size_t(iso)));
   tri_bisect(ctx, f.w->as<double>(), f.e->as<double>(), int(iso), 0, int(iso), f.lam->as<double>());
   f.wh = static_cast<double*>(stage_take(ctx, sizeof(double) * size_t(iso)));
@@ -337,8 +346,10 @@ void fact_tri_solve(nsmi_ctx* ctx, FactCore& f) {
 // svd route: the isometry side as a tall matrix X (its left singular vectors, or its
 // right ones when the isometry side is the shorter one), bidiagonalised in one launch,
 // then the singular values by bisection on the Golub-Kahan matrix (descending),
-// copied to the host.  False, with nothing launched, beyond the kernel's range.
-bool fact_svd_launch(nsmi_ctx* ctx, FactCore& f) {
+// copied to the host.  False, with nothing launched, beyond the kernel's range.  spread: as
+// for the reduction's launch.
+bool fact_svd_launch(nsmi_ctx* ctx, FactCore& f, bool spread = false) {
+  f.bid = false;
   const int64_t m = f.m, nc = f.nc;
   f.want_v = f.iso < f.oth;
   const bool x_is_m = f.rows_trailing ? (nc < m) : (m >= nc);
@@ -359,7 +370,7 @@ bool fact_svd_launch(nsmi_ctx* ctx, FactCore& f) {
   f.tau.reset(new Scratch(ctx, sizeof(double) * size_t(s)));
   f.tauR.reset(new Scratch(ctx, sizeof(double) * size_t(std::max(s - 1, 1))));
   if (!bidiag_launch(ctx, f.X->as<double>(), r, s, f.w->as<double>(), f.e->as<double>(), f.tau->as<double>(),
-                     f.tauR->as<double>(), f.sr)) {
+                     f.tauR->as<double>(), f.sr, spread)) {
     f.X.reset();
     return false;
   }
@@ -464,8 +475,13 @@ void fact_jacobi(nsmi_ctx* ctx, const std::vector<FactCore*>& fs) {
 
 void fact_prepare(nsmi_ctx* ctx, FactCore& f) {
   if (f.route == NSMI_ROUTE_SVD) {
-    if (fact_svd_launch(ctx, f)) {
-      NSMI_HIP(hipStreamSynchronize(ctx->stream));
+    bool launched = fact_svd_launch(ctx, f);
+    if (launched) NSMI_HIP(hipStreamSynchronize(ctx->stream));
+    for (int i = 0; i < kRelaunches && launched && reduction_unplaced(f.sr); ++i) {
+      launched = fact_svd_launch(ctx, f, true);
+      if (launched) NSMI_HIP(hipStreamSynchronize(ctx->stream));
+    }
+    if (launched) {
       fact_finish(f);
       return;
     }

@@ -26,18 +26,11 @@
 
 #include <type_traits>
 
+#include "internal.h"
 #include "wave.h"
 
 namespace nsmi {
 namespace {
-
-constexpr int kXcds = 8;
-
-// control words of a reduction (zero on entry): the flags the host reads, then the
-// counters, each on its own 128-byte line
-constexpr int kCtlFail = 32, kCtlNonFinite = 33;     // host-visible flags
-constexpr int kCtlArrived = 64, kCtlTicket = 96;     // placement: all workgroups, one ticket line per XCD
-constexpr int kCtlWords = kCtlTicket + 32 * kXcds;
 
 // the empty word: a signalling NaN's pattern (arithmetic only makes quiet ones)
 constexpr unsigned long long kEmpty = 0x7FF4C0DE5EED0001ull;
@@ -99,72 +92,70 @@ __device__ __forceinline__ bool load_words(double (&v)[N], const Addr& addr, uns
   }
 }
 
-// bounded wait by one lane until *p reaches target; false (with the failure flag
-// raised) when it gives up or another workgroup has
-__device__ inline bool wait_reach(const unsigned* p, unsigned target, unsigned* fail) {
-  for (unsigned spins = 0; ld_agent(p) < target; ++spins) {
-    if ((spins & 255u) == 255u && ld_agent(fail) != 0u) return false;
-    if (spins > (1u << 22)) {
-      atomicOr(fail, 1u);
-      return false;
-    }
+// ---- placement.  No workgroup of a group does any work before the group's placement is
+// decided, once, by a compare-and-swap of kCtlPlaced from 0: placed when all of the group's
+// workgroups are on the device, unplaced when that cannot be or takes too long; then all of
+// them leave, nothing has been written, and the host launches again.  So a group that is
+// only partly resident never holds its CUs for good.
+__device__ inline void decide(unsigned* ctl, unsigned state) {
+  unsigned undecided = 0u;
+  __hip_atomic_compare_exchange_strong(ctl + kCtlPlaced, &undecided, state, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+  stores_done();
+}
+// one lane's wait for the decision, about half a second at most
+__device__ inline bool placed(unsigned* ctl) {
+  for (unsigned spins = 0;; ++spins) {
+    const unsigned state = ld_agent(ctl + kCtlPlaced);
+    if (state != 0u) return state == kPlaced;
+    if (spins == (1u << 20)) decide(ctl, kUnplaced);
   }
-  return true;
 }
 
-// Placement of a one-group launch: the grid holds 8 G workgroups, of which G on the
-// wanted XCD form the group (their tickets give the order) and the others leave.  The
-// dispatcher hands workgroups out to the XCDs in turn, so the wanted one gets G; if
-// it does not, the first G workgroups of the grid form the group and exchange past L2
-// (local = false).  Returns the workgroup's index in the group, -1 to leave.
-__device__ inline int place_one_xcd(unsigned* ctl, int G, int want, bool* local, int* s_place) {
+// Placement of a group on XCD `want`: the grid holds 8 G workgroups, of which the first G on
+// that XCD (their tickets give the order) form the group.  All the others leave at once:
+// they must not keep their CUs, where the members of other groups may be waiting to start.
+// The dispatcher hands workgroups out to the XCDs in turn, so the wanted one gets G; if every
+// workgroup has arrived and it did not, the last one to arrive says so.  Returns the
+// workgroup's index in the group, -1 to leave.
+__device__ inline int place_one_xcd(unsigned* ctl, int G, int want, int* s_place) {
   if (threadIdx.x == 0) {
-    const unsigned total = gridDim.x;
-    unsigned* const fail = ctl + kCtlFail;
-    unsigned* const tick = ctl + kCtlTicket + 32 * want;
-    const bool mine = xcd_id() == want;
-    const unsigned t = mine ? add_agent(tick) : 0u;
-    stores_done();
-    add_agent(ctl + kCtlArrived);
     int place = -1;
-    bool full = false;
-    for (unsigned spins = 0;; ++spins) {
-      full = ld_agent(tick) >= unsigned(G);
-      if (full) break;
-      if (ld_agent(ctl + kCtlArrived) >= total) {  // every ticket is taken
-        full = ld_agent(tick) >= unsigned(G);
-        break;
-      }
-      if (spins > (1u << 22)) {
-        atomicOr(fail, 1u);
-        break;
-      }
+    if (xcd_id() == want) {
+      const unsigned t = add_agent(ctl + kCtlTicket + 32 * want);
+      if (t < unsigned(G)) place = int(t);
+      if (t == unsigned(G) - 1u) decide(ctl, kPlaced);
     }
-    if (full)
-      place = mine && t < unsigned(G) ? int(t) : -1;
-    else
-      place = int(blockIdx.x) < G ? (int(blockIdx.x) | (1 << 30)) : -1;
+    if (add_agent(ctl + kCtlArrived) == gridDim.x - 1u) decide(ctl, kUnplaced);
+    if (place >= 0 && !placed(ctl)) place = -1;
     *s_place = place;
   }
   __syncthreads();
-  const int place = __builtin_amdgcn_readfirstlane(*s_place);
-  *local = place < 0 || !(place & (1 << 30));
-  return place < 0 ? -1 : (place & ~(1 << 30));
+  return __builtin_amdgcn_readfirstlane(*s_place);
+}
+
+// Placement of a group wherever its workgroups are, in the grid's order.
+__device__ inline int place_spread(unsigned* ctl, int* s_place) {
+  if (threadIdx.x == 0) {
+    if (add_agent(ctl + kCtlArrived) == gridDim.x - 1u) decide(ctl, kPlaced);
+    *s_place = placed(ctl) ? int(blockIdx.x) : -1;
+  }
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(*s_place);
 }
 
 // Placement of a launch over all XCDs, 8 GW workgroups: XCD x and index w inside it.
-// Where the dispatcher did not hand GW workgroups to each XCD the groups are formed by
-// the grid index instead (local = false).
-__device__ inline bool place_all_xcds(unsigned* ctl, int GW, int* x, int* w, bool* local, int* s_place) {
+// Where the dispatcher did not hand GW workgroups to each XCD (or the host asks for it,
+// want < 0) the groups are formed by the grid index instead (local = false).
+__device__ inline bool place_all_xcds(unsigned* ctl, int GW, int want, int* x, int* w, bool* local, int* s_place) {
   if (threadIdx.x == 0) {
-    unsigned* const fail = ctl + kCtlFail;
     const int xc = xcd_id();
     const unsigned t = add_agent(ctl + kCtlTicket + 32 * xc);
     stores_done();
-    add_agent(ctl + kCtlArrived);
+    if (add_agent(ctl + kCtlArrived) == gridDim.x - 1u) decide(ctl, kPlaced);
     int p = -1;
-    if (wait_reach(ctl + kCtlArrived, gridDim.x, fail)) {
-      bool even = true;
+    if (placed(ctl)) {
+      bool even = want >= 0;
       for (int q = 0; q < kXcds; ++q) even = even && ld_agent(ctl + kCtlTicket + 32 * q) == unsigned(GW);
       p = even ? int(t) * kXcds + xc : (int(blockIdx.x) | (1 << 30));
     }

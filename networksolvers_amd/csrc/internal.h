@@ -159,6 +159,8 @@ struct nsmi_ctx {
   nsmi_profile_stats stats[NSMI_K_COUNT] = {};
   // multi-workgroup reductions still to start with the timeout flag raised (tests)
   int inject_timeouts = 0;
+  // placements of multi-workgroup reductions still to fail (tests)
+  int inject_misplaced = 0;
   // while set (nsmi_heff_apply_noalloc), split-K GEMMs take their partial sums from
   // this device buffer instead of the pool, and fail when it is too small
   void* fixed_part = nullptr;
@@ -424,17 +426,41 @@ void small_sym_eigh(int n, const double* A, double* w, double* V);  // host Jaco
 // LAPACK's dsytrd "lower" order, reflectors in place (one launch); false when n is outside
 // [2, kSytrdMax] or the device cannot co-schedule the grid.
 constexpr int kSytrdMax = 1024;
-// one asynchronous tridiagonal reduction: its exchange and flag buffers, and the
-// host copy of the two failure flags (an exchange that timed out, non-finite d or e)
+//
+// Control words of a reduction (zero on entry): the words the host reads (an exchange that
+// timed out, non-finite d or e, the state of the placement), then the counters of the
+// placement, each on its own 128-byte line (all workgroups, one ticket line per XCD).
+constexpr int kXcds = 8;
+constexpr int kCtlFail = 32, kCtlNonFinite = 33, kCtlPlaced = 34, kCtlHostWords = 3;
+constexpr int kCtlArrived = 64, kCtlTicket = 96;
+constexpr int kCtlWords = kCtlTicket + 32 * kXcds;
+constexpr unsigned kPlaced = 1, kUnplaced = 2;  // kCtlPlaced once it is decided (group.h)
+// one asynchronous reduction: its exchange and control words, and the host copy of
+// kCtlHostWords of them from kCtlFail on
 struct SytrdRun {
   std::unique_ptr<Scratch> xch, flags;
-  unsigned* host_flags = nullptr;  // two flags in pinned stage memory
+  unsigned* host_flags = nullptr;  // in pinned stage memory
 };
-bool sytrd_launch(nsmi_ctx* ctx, double* A, int n, double* d, double* e, double* tau, SytrdRun& run);
+// spread: the workgroups of a group go wherever there is room and not to one XCD
+bool sytrd_launch(nsmi_ctx* ctx, double* A, int n, double* d, double* e, double* tau, SytrdRun& run,
+                  bool spread = false);
+// Whether groups of up to 32 workgroups on one XCD can be asked for on this device
+bool one_xcd_groups(nsmi_ctx* ctx);
 // runs launch(xcd) for a kernel whose group of at most 32 workgroups (two of them to a CU)
 // runs on one XCD: the stream's place among the XCDs, see bidiag.hip
 void launch_on_one_xcd(nsmi_ctx* ctx, const std::function<void(int)>& launch);
 void xcd_places_release(int device, hipStream_t stream);
+// whether a placement is to fail, by injection (tests); counts it
+bool take_misplacement(nsmi_ctx* ctx);
+// cooperative launch of a group that needs all of its grid resident; false, with nothing
+// launched, when the device cannot
+bool launch_cooperative(nsmi_ctx* ctx, const void* fn, int groups, int threads, void** args);
+// enqueues the host copy of a launched reduction's control words
+void reduction_readback(nsmi_ctx* ctx, SytrdRun& run);
+// once the copy has arrived: whether the group never started (nothing written; launch again,
+// spread, kRelaunches times)
+constexpr int kRelaunches = 2;
+inline bool reduction_unplaced(const SytrdRun& run) { return run.host_flags[kCtlPlaced - kCtlFail] == kUnplaced; }
 // start value of a reduction's failure flag: 1 when the context has an injected timeout
 // pending and the grid has G > 1
 unsigned reduction_fail0(nsmi_ctx* ctx, int G);
@@ -451,13 +477,13 @@ void apply_reflectors(nsmi_ctx* ctx, const double* Vt, const double* tau, int m,
 // ---- own dense SVD / tridiagonal eigensolver pieces (svd.hip) -------------------
 // One-launch Householder bidiagonalisation of a tall r x s device matrix X (r >= s,
 // row-major; reflectors left in place, see bidiag.h), d (s), e, tauR (s - 1), tauL (s).
-// Enqueues the launch and the copy of its two failure flags (as sytrd_launch); false
+// Enqueues the launch and the copy of its control words (as sytrd_launch); false
 // with nothing launched when the size is outside the kernels' range or the grid cannot
 // be co-scheduled.
 constexpr int kBidiagMax = 2048, kBidiagRowsMax = 4096;
 int bidiag_groups(int r, int s);
 bool bidiag_launch(nsmi_ctx* ctx, double* X, int r, int s, double* d, double* e, double* tauL, double* tauR,
-                   SytrdRun& run);
+                   SytrdRun& run, bool spread = false);
 // the Golub-Kahan off-diagonal (d_0, e_0, d_1, ..., d_{s-1}) of the bidiagonal (2 s - 1 entries)
 void gk_offdiag(nsmi_ctx* ctx, const double* d, const double* e, int s, double* gk);
 // eigenvalues of descending rank i0 .. i0 + count - 1 of the symmetric tridiagonal

@@ -42,16 +42,13 @@ __global__ __launch_bounds__(64 * NW, CL > 8 ? 1 : NW / 2) void k_sytrd(
   __shared__ double vl[NW][NP];                           // each wave's v, by column
   __shared__ double ps[SHARED ? NP : 1], yv[SHARED ? NP : 1];
   __shared__ int s_ok, s_place;
+  static_assert(CL > 8 || sizeof(vl) + sizeof(ps) + sizeof(yv) < 160 * 1024 / 3,
+                "two workgroups of one-XCD groups share a CU");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   unsigned* const fail = ctl + kCtlFail;
-  bool local = true;
-  int g = blockIdx.x;
-  if (want >= 0) {
-    g = place_one_xcd(ctl, G, want, &local, &s_place);
-    if (g < 0) return;
-  } else {
-    local = false;  // a group over all XCDs: the words go past L2
-  }
+  const bool local = want >= 0;  // else a group over all XCDs: the words go past L2
+  const int g = local ? place_one_xcd(ctl, G, want, &s_place) : place_spread(ctl, &s_place);
+  if (g < 0) return;
   double* const P = xch;            // [3][SP]
   double* const Y = xch + 3 * SP;   // [3][SP]
 

@@ -105,3 +105,95 @@ def test_reductions_on_more_streams_than_places(ctx):
     assert not errors
     for i in range(18):
         np.testing.assert_array_equal(got[i], want)
+
+
+def _reduce_launches(ctx, fn):
+    """fn() with the reductions' launches counted."""
+    ctx.profile(True)
+    ctx.profile_reset()
+    out = fn()
+    n = ctx.profile_stats()["fact_reduce"]["launches"]
+    ctx.profile(False)
+    return out, n
+
+
+@pytest.mark.parametrize("m,n,route", [(60, 64, "svd"), (128, 100, "svd"), (300, 70, "svd"), (300, 280, "svd"),
+                                       (512, 500, "svd"), (700, 520, "svd"), (64, 90, "eigen"), (130, 140, "eigen"),
+                                       (300, 310, "eigen"), (512, 520, "eigen")])
+def test_misplaced_groups_give_the_same_result(ctx, m, n, route):
+    """A group that does not get the XCD it asks for leaves without having started and is
+    launched again over the whole device (up to 512 columns and rows); one over all XCDs (700 x
+    520) is formed in the grid's order.  Every sum has a fixed order, so the factors are the
+    same bit for bit."""
+    import networksolvers_amd as ns
+    x = ctx.upload(np.random.default_rng(m + n).standard_normal((m, n)))
+    print(f"misplaced m={m} n={n} route={route}", flush=True)
+
+    def run():
+        U, C, info = ns.factorize(x, 1, False, cutoff=1e-10, maxdim=20, which_decomp=route)
+        return U.numpy(), C.numpy(), info.route
+    (u, c, r), once = _reduce_launches(ctx, run)
+    ctx.check(ctx.lib.nsmi_inject_misplacement(ctx.h, 1))
+    (u1, c1, r1), twice = _reduce_launches(ctx, run)
+    assert once == 1 and twice == (1 if m == 700 else 2) and r == r1
+    np.testing.assert_array_equal(u, u1)
+    np.testing.assert_array_equal(c, c1)
+
+
+def test_misplaced_sector_groups_give_the_same_result(ctx):
+    """Three of six sectors' groups, on four streams, are launched again; the sectors' factors
+    are the same bit for bit."""
+    from networksolvers_amd import qn
+    shapes = [(80, 90), (60, 70), (300, 200), (30, 35), (150, 149), (45, 200)]
+    rng = np.random.default_rng(5)
+    offs = np.concatenate([[0], np.cumsum([m * n for m, n in shapes])])[:-1].tolist()
+    buf = ctx.upload(rng.standard_normal(sum(m * n for m, n in shapes)))
+    rows, cols = [m for m, _ in shapes], [n for _, n in shapes]
+
+    def run():
+        U, C, kept, _ = qn._factorize_sectors(ctx, buf, offs, rows, cols, False, 1e-10, 100, 1, "eigen")
+        return U.numpy(), C.numpy(), kept
+    (u, c, k), once = _reduce_launches(ctx, run)
+    print("misplaced sectors", flush=True)
+    ctx.check(ctx.lib.nsmi_inject_misplacement(ctx.h, 3))
+    (u1, c1, k1), more = _reduce_launches(ctx, run)
+    assert (once, more) == (5, 8) and k == k1
+    np.testing.assert_array_equal(u, u1)
+    np.testing.assert_array_equal(c, c1)
+
+
+def test_full_groups_of_many_streams_at_once(ctx):
+    """Groups of up to 32 workgroups that fill half of an XCD each (four waves of 256 registers,
+    n = 500 on the eigen route; eight of 128, 500 x 490 on the svd route), from ten contexts on
+    five threads, several of them in flight at any time on places of the same XCD: every
+    result equals the first context's, bit for bit."""
+    import threading
+
+    import networksolvers_amd as ns
+    rng = np.random.default_rng(4)
+    work = [(rng.standard_normal((500, 510)), "eigen"), (rng.standard_normal((500, 490)), "svd"),
+            (rng.standard_normal((1000, 120)), "svd")]
+    ctxs = [ns.Context(0) for _ in range(10)]
+
+    def run(c, M, route):
+        return ns.factorize(c.upload(M), 1, False, cutoff=0.0, maxdim=20, which_decomp=route)[1].numpy()
+    want = [run(ctx, M, route) for M, route in work]
+    errors = []
+
+    def worker(t):
+        try:
+            for it in range(4):
+                for i in range(t, 10, 5):
+                    j = (t + it + i) % len(work)
+                    np.testing.assert_array_equal(run(ctxs[i], *work[j]), want[j])
+        except BaseException as ex:   # noqa: BLE001
+            errors.append(ex)
+    ts = [threading.Thread(target=worker, args=(t,)) for t in range(5)]
+    print("full groups of ten streams", flush=True)
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for c in ctxs:
+        c.close()
+    assert not errors, errors
