@@ -6,58 +6,64 @@
 #include <mutex>
 
 #include "internal.h"
+#include "places.h"
 
 namespace nsmi {
 namespace {
 
-// Two groups at a time may hold an XCD (kGroupsPerXcd: their workgroups, at most one for
-// each of its CUs, fit two to a CU, and nothing but their members stays on the device, see
-// place_one_xcd), so both become resident; with a third one each could have a part of its
-// CUs and none enough.  Each stream that launches such groups is given one of the 16 places
-// (8 XCDs x 2) for its life, spread over the XCDs first.  With more than 16 streams a place
-// is shared: a launch then waits for what the others sharing it have queued (an event per
-// stream, under the lock, so that two of them cannot pass each other).
-constexpr int kCusPerXcd = 32, kGroupsPerXcd = 2;
-struct XcdPlaces {
+struct DevicePlaces {
   std::mutex mu;
-  std::vector<hipStream_t> users[kGroupsPerXcd * kXcds];
-  hipEvent_t ev = nullptr;
+  XcdPlaces<hipStream_t> places;
+  hipEvent_t ev = nullptr;         // for the waits on streams
+  hipEvent_t device_ev = nullptr;  // the last group over the device
 };
-XcdPlaces& places_of(int device) {
+DevicePlaces& places_of(int device) {
   static std::mutex mu;
-  static std::map<int, XcdPlaces> all;
+  static std::map<int, DevicePlaces> all;
   std::lock_guard<std::mutex> lock(mu);
   return all[device];
+}
+
+void wait_in_order(nsmi_ctx* ctx, DevicePlaces& p, const XcdPlaces<hipStream_t>::Order& o) {
+  for (hipStream_t s : o.streams) {
+    if (!p.ev) NSMI_HIP(hipEventCreateWithFlags(&p.ev, hipEventDisableTiming));
+    NSMI_HIP(hipEventRecord(p.ev, s));
+    NSMI_HIP(hipStreamWaitEvent(ctx->stream, p.ev, 0));
+  }
+  if (o.device && p.device_ev) NSMI_HIP(hipStreamWaitEvent(ctx->stream, p.device_ev, 0));
 }
 
 }  // namespace
 
 void launch_on_one_xcd(nsmi_ctx* ctx, const std::function<void(int)>& launch) {
-  XcdPlaces& p = places_of(ctx->device);
+  DevicePlaces& p = places_of(ctx->device);
   std::lock_guard<std::mutex> lock(p.mu);
-  int at = -1, best = 0;
-  for (int i = 0; i < kGroupsPerXcd * kXcds; ++i) {
-    for (hipStream_t s : p.users[i])
-      if (s == ctx->stream) at = i;
-    if (p.users[i].size() < p.users[best].size()) best = i;
-  }
-  if (at < 0) {
-    p.users[best].push_back(ctx->stream);
-    at = best;
-  }
-  for (hipStream_t s : p.users[at]) {
-    if (s == ctx->stream) continue;
-    if (!p.ev) NSMI_HIP(hipEventCreateWithFlags(&p.ev, hipEventDisableTiming));
-    NSMI_HIP(hipEventRecord(p.ev, s));
-    NSMI_HIP(hipStreamWaitEvent(ctx->stream, p.ev, 0));
-  }
-  launch(at % kXcds);
+  const auto o = p.places.one_xcd(ctx->stream);
+  wait_in_order(ctx, p, o);
+  launch(o.xcd);
+}
+
+bool launch_over_device(nsmi_ctx* ctx, const void* fn, int groups, int threads, void** args) {
+  int coop = 0, ncu = 0, per_cu = 0;
+  NSMI_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device));
+  NSMI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
+  NSMI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, 0));
+  if (!coop || per_cu < 1 || groups > ncu * per_cu) return false;
+  DevicePlaces& p = places_of(ctx->device);
+  std::lock_guard<std::mutex> lock(p.mu);
+  if (!p.device_ev) NSMI_HIP(hipEventCreateWithFlags(&p.device_ev, hipEventDisableTiming));
+  wait_in_order(ctx, p, p.places.over_device(ctx->stream));
+  const hipError_t st = hipLaunchCooperativeKernel(fn, dim3(unsigned(groups)), dim3(unsigned(threads)), args, 0,
+                                                   ctx->stream);
+  if (st != hipSuccess) (void)hipGetLastError();
+  NSMI_HIP(hipEventRecord(p.device_ev, ctx->stream));
+  return st == hipSuccess;
 }
 
 void xcd_places_release(int device, hipStream_t stream) {
-  XcdPlaces& p = places_of(device);
+  DevicePlaces& p = places_of(device);
   std::lock_guard<std::mutex> lock(p.mu);
-  for (auto& u : p.users) u.erase(std::remove(u.begin(), u.end(), stream), u.end());
+  p.places.release(stream);
 }
 
 unsigned reduction_fail0(nsmi_ctx* ctx, int G) {
@@ -76,19 +82,7 @@ bool one_xcd_groups(nsmi_ctx* ctx) {
   int xcds = 0, ncu = 0;
   NSMI_HIP(hipDeviceGetAttribute(&xcds, hipDeviceAttributeNumberOfXccs, ctx->device));
   NSMI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
-  return xcds == kXcds && ncu >= kXcds * kCusPerXcd;
-}
-
-bool launch_cooperative(nsmi_ctx* ctx, const void* fn, int groups, int threads, void** args) {
-  int coop = 0, ncu = 0, per_cu = 0;
-  NSMI_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device));
-  NSMI_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
-  NSMI_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, 0));
-  if (!coop || per_cu < 1 || groups > ncu * per_cu) return false;
-  const hipError_t st = hipLaunchCooperativeKernel(fn, dim3(unsigned(groups)), dim3(unsigned(threads)), args, 0,
-                                                   ctx->stream);
-  if (st != hipSuccess) (void)hipGetLastError();
-  return st == hipSuccess;
+  return xcds == kXcds && ncu >= kXcds * XcdPlaces<hipStream_t>::kCusPerXcd;
 }
 
 void reduction_readback(nsmi_ctx* ctx, SytrdRun& run) {
@@ -108,7 +102,8 @@ struct BidiagPlan {
 };
 template <int CL, int RW, int NW, BidiagMode MODE, int GMAX>
 BidiagPlan plan_of() {
-  static_assert(MODE == kOneGroup || GMAX <= kCusPerXcd, "at most one workgroup for each CU of an XCD");
+  static_assert(MODE == kOneGroup || GMAX <= XcdPlaces<hipStream_t>::kCusPerXcd,
+                "at most one workgroup for each CU of an XCD");
   return {reinterpret_cast<const void*>(k_bidiag<CL, RW, NW, MODE, GMAX>), MODE, CL, 64 * NW, GMAX, RW * NW};
 }
 
@@ -123,7 +118,7 @@ BidiagPlan plan_of() {
 //   with 16 workgroups of twice the rows), 2.9 at 1000 x 256, 3.7 at 2000 x 128;
 //   all XCDs: 3.7 at 512 x 512, 4.2 at 700 x 700, 4.5 at 1000 x 1000 (5.2 on one XCD), 5.9 at
 //   2048 x 2048, 5.8 at 4000 x 1000.
-// One-XCD groups go out as ordinary launches (at most 32 workgroups, places_of); the
+// One-XCD groups go out as ordinary launches (at most 32 workgroups, places.h); the
 // others need up to one workgroup on every CU and take the cooperative launch, and so does a
 // one-XCD group that was not placed or that the device has no XCDs for.
 BidiagPlan bidiag_plan(int r, int s) {
@@ -198,7 +193,7 @@ bool bidiag_launch(nsmi_ctx* ctx, double* X, int r, int s, double* d, double* e,
       NSMI_HIP(hipLaunchKernel(p.fn, dim3(1), dim3(unsigned(p.threads)), args, 0, ctx->stream));
     } else if (p.mode == kAllXcds || spread || !one_xcd_groups(ctx)) {
       if (p.mode == kAllXcds && !take_misplacement(ctx)) want = 0;
-      if (!launch_cooperative(ctx, p.fn, G, p.threads, args)) return false;
+      if (!launch_over_device(ctx, p.fn, G, p.threads, args)) return false;
     } else {
       launch_on_one_xcd(ctx, [&](int xcd) {
         want = take_misplacement(ctx) ? kXcds : xcd;  // kXcds: none has this number

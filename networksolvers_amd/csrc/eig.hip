@@ -317,7 +317,7 @@ bool sytrd_launch(nsmi_ctx* ctx, double* A, int n, double* d, double* e, double*
   {
     ProfScope ps(ctx, NSMI_K_FACT_REDUCE, 4.0 / 3.0 * double(n) * n * n, 16.0 * double(n) * n);
     if (p.spread || spread || !one_xcd_groups(ctx)) {
-      if (!launch_cooperative(ctx, p.fn, G, p.threads, args)) return false;
+      if (!launch_over_device(ctx, p.fn, G, p.threads, args)) return false;
     } else {
       launch_on_one_xcd(ctx, [&](int xcd) {
         want = take_misplacement(ctx) ? kXcds : xcd;  // kXcds: none has this number

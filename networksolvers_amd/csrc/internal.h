@@ -447,14 +447,14 @@ bool sytrd_launch(nsmi_ctx* ctx, double* A, int n, double* d, double* e, double*
 // Whether groups of up to 32 workgroups on one XCD can be asked for on this device
 bool one_xcd_groups(nsmi_ctx* ctx);
 // runs launch(xcd) for a kernel whose group of at most 32 workgroups (two of them to a CU)
-// runs on one XCD: the stream's place among the XCDs, see bidiag.hip
+// runs on one XCD: the stream's place among the XCDs, see places.h
 void launch_on_one_xcd(nsmi_ctx* ctx, const std::function<void(int)>& launch);
 void xcd_places_release(int device, hipStream_t stream);
 // whether a placement is to fail, by injection (tests); counts it
 bool take_misplacement(nsmi_ctx* ctx);
-// cooperative launch of a group that needs all of its grid resident; false, with nothing
-// launched, when the device cannot
-bool launch_cooperative(nsmi_ctx* ctx, const void* fn, int groups, int threads, void** args);
+// cooperative launch of a group over the device, alone among the groups (places.h); false, with
+// nothing launched, when the device cannot hold all of its grid
+bool launch_over_device(nsmi_ctx* ctx, const void* fn, int groups, int threads, void** args);
 // enqueues the host copy of a launched reduction's control words
 void reduction_readback(nsmi_ctx* ctx, SytrdRun& run);
 // once the copy has arrived: whether the group never started (nothing written; launch again,

@@ -162,18 +162,12 @@ def test_misplaced_sector_groups_give_the_same_result(ctx):
     np.testing.assert_array_equal(c, c1)
 
 
-def test_full_groups_of_many_streams_at_once(ctx):
-    """Groups of up to 32 workgroups that fill half of an XCD each (four waves of 256 registers,
-    n = 500 on the eigen route; eight of 128, 500 x 490 on the svd route), from ten contexts on
-    five threads, several of them in flight at any time on places of the same XCD: every
-    result equals the first context's, bit for bit."""
+def _same_from_threads(ctx, ctxs, work, rounds):
+    """Every context factorises the matrices of `work` in turn, five threads sharing the
+    contexts; C is compared with that of `ctx` alone."""
     import threading
 
     import networksolvers_amd as ns
-    rng = np.random.default_rng(4)
-    work = [(rng.standard_normal((500, 510)), "eigen"), (rng.standard_normal((500, 490)), "svd"),
-            (rng.standard_normal((1000, 120)), "svd")]
-    ctxs = [ns.Context(0) for _ in range(10)]
 
     def run(c, M, route):
         return ns.factorize(c.upload(M), 1, False, cutoff=0.0, maxdim=20, which_decomp=route)[1].numpy()
@@ -182,18 +176,47 @@ def test_full_groups_of_many_streams_at_once(ctx):
 
     def worker(t):
         try:
-            for it in range(4):
-                for i in range(t, 10, 5):
+            for it in range(rounds):
+                for i in range(t, len(ctxs), 5):
                     j = (t + it + i) % len(work)
                     np.testing.assert_array_equal(run(ctxs[i], *work[j]), want[j])
         except BaseException as ex:   # noqa: BLE001
             errors.append(ex)
     ts = [threading.Thread(target=worker, args=(t,)) for t in range(5)]
-    print("full groups of ten streams", flush=True)
     for t in ts:
         t.start()
     for t in ts:
         t.join()
+    assert not errors, errors
+
+
+def test_full_groups_of_many_streams_at_once(ctx):
+    """Groups of up to 32 workgroups that fill half of an XCD each (four waves of 256 registers,
+    n = 500 on the eigen route; eight of 128, 500 x 490 on the svd route), from ten contexts on
+    five threads, several of them in flight at any time on places of the same XCD: every
+    result equals the first context's, bit for bit."""
+    import networksolvers_amd as ns
+    rng = np.random.default_rng(4)
+    work = [(rng.standard_normal((500, 510)), "eigen"), (rng.standard_normal((500, 490)), "svd"),
+            (rng.standard_normal((1000, 120)), "svd")]
+    ctxs = [ns.Context(0) for _ in range(10)]
+    print("full groups of ten streams", flush=True)
+    _same_from_threads(ctx, ctxs, work, 4)
     for c in ctxs:
         c.close()
-    assert not errors, errors
+
+
+def test_groups_over_the_device_beside_groups_of_one_xcd(ctx):
+    """Contexts on five threads mix groups over all XCDs (1100 x 520 and 700 x 700 on the svd
+    route, n = 600 on the eigen route) with groups that fill half of an XCD: every result
+    equals the first context's, bit for bit."""
+    import networksolvers_amd as ns
+    rng = np.random.default_rng(6)
+    work = [(rng.standard_normal((1100, 520)), "svd"), (rng.standard_normal((500, 490)), "svd"),
+            (rng.standard_normal((700, 700)), "svd"), (rng.standard_normal((500, 510)), "eigen"),
+            (rng.standard_normal((600, 610)), "eigen")]
+    ctxs = [ns.Context(0) for _ in range(10)]
+    print("groups over the device beside groups of one XCD", flush=True)
+    _same_from_threads(ctx, ctxs, work, 5)
+    for c in ctxs:
+        c.close()
