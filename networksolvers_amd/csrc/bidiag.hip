@@ -2,6 +2,8 @@
 // its one-XCD groups run on.
 #include "bidiag.h"
 
+#include <unistd.h>
+
 #include <algorithm>
 #include <mutex>
 
@@ -13,7 +15,7 @@ namespace {
 
 struct DevicePlaces {
   std::mutex mu;
-  XcdPlaces<hipStream_t> places;
+  XcdPlaces<hipStream_t> places{unsigned(getpid())};
   hipEvent_t ev = nullptr;         // for the waits on streams
   hipEvent_t device_ev = nullptr;  // the last group over the device
 };

@@ -459,7 +459,7 @@ bool launch_over_device(nsmi_ctx* ctx, const void* fn, int groups, int threads, 
 void reduction_readback(nsmi_ctx* ctx, SytrdRun& run);
 // once the copy has arrived: whether the group never started (nothing written; launch again,
 // spread, kRelaunches times)
-constexpr int kRelaunches = 2;
+constexpr int kRelaunches = 4;
 inline bool reduction_unplaced(const SytrdRun& run) { return run.host_flags[kCtlPlaced - kCtlFail] == kUnplaced; }
 // start value of a reduction's failure flag: 1 when the context has an injected timeout
 // pending and the grid has G > 1

@@ -15,6 +15,11 @@
 //   * one-XCD: for the other streams of its place, and for the last group over the device;
 //   * over the device: for every stream that launched a one-XCD group since the last group
 //     over the device, and for that one.
+// Other processes on the device are not seen.  Each starts its places at an XCD of its own
+// (first), so that a few processes of few streams each stay apart; where too many groups meet all
+// the same, the placement ends without a group having started and it is launched again
+// (group.h).
+//
 // The caller holds a lock from the question to its launch, so launches are ordered as they
 // asked and never wait in a circle.  Host code without HIP, tested as such.
 #pragma once
@@ -33,6 +38,8 @@ class XcdPlaces {
     bool device = false;          // wait for the last group over the device
   };
 
+  explicit XcdPlaces(unsigned first = 0) : first_(first) {}
+
   Order one_xcd(Stream s) {
     int at = -1, best = 0;
     for (int i = 0; i < kPlaces; ++i) {
@@ -45,7 +52,7 @@ class XcdPlaces {
       users_[at].push_back(User{s, false});
     }
     Order o;
-    o.xcd = at % kXcdCount;
+    o.xcd = int((unsigned(at) + first_) % kXcdCount);
     for (User& u : users_[at]) {
       if (u.s == s)
         u.active = true;
@@ -81,6 +88,7 @@ class XcdPlaces {
     Stream s;
     bool active;  // a one-XCD group launched since the last group over the device
   };
+  unsigned first_;
   std::vector<User> users_[kPlaces];
   Stream device_stream_{};
   bool device_busy_ = false;

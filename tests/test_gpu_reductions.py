@@ -220,3 +220,54 @@ def test_groups_over_the_device_beside_groups_of_one_xcd(ctx):
     _same_from_threads(ctx, ctxs, work, 5)
     for c in ctxs:
         c.close()
+
+
+_PROCESS = """
+import sys
+import numpy as np
+import networksolvers_amd as ns
+seed = int(sys.argv[1])
+ctx = ns.Context(0)
+rng = np.random.default_rng(seed)
+work = [(rng.standard_normal((500, 490)), "svd"), (rng.standard_normal((500, 510)), "eigen"),
+        (rng.standard_normal((150, 140)), "svd"), (rng.standard_normal((700, 600)), "svd")]
+print("ready", flush=True)
+sys.stdin.readline()
+for it in range(8):
+    for M, route in work:
+        C = ns.factorize(ctx.upload(M), 1, False, cutoff=0.0, maxdim=20, which_decomp=route)[1].numpy()
+        s = np.linalg.svd(M, compute_uv=False) if it == 0 else None
+        if it == 0:
+            assert np.abs(np.linalg.norm(C, axis=1) - s[:20]).max() < 1e-12 * s[0]
+            first = globals().setdefault("first", {})
+            first[M.shape] = C
+        assert np.array_equal(C, first[M.shape])
+ctx.close()
+"""
+
+
+def test_groups_of_several_processes(ctx):
+    """Three processes, started together, factorise at the same time, with groups that fill half
+    of an XCD and groups over all of them; none knows of the others' launches."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, OMP_NUM_THREADS="4")
+    procs = [subprocess.Popen([sys.executable, "-c", _PROCESS, str(seed)], cwd=root, env=env, text=True,
+                              stdin=subprocess.PIPE, stdout=subprocess.PIPE, stderr=subprocess.PIPE)
+             for seed in range(3)]
+    try:
+        for p in procs:
+            assert p.stdout.readline().strip() == "ready"
+        print("three processes", flush=True)
+        for p in procs:
+            p.stdin.write("go\n")
+            p.stdin.flush()
+        for p in procs:
+            _, err = p.communicate(timeout=60)
+            assert p.returncode == 0, err[-2000:]
+    finally:
+        for p in procs:
+            if p.poll() is None:
+                p.kill()

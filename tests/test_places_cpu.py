@@ -20,7 +20,9 @@ using Past = std::bitset<N>;                 // launches that have ended before 
 int main(int argc, char** argv) {
   const int seed = std::atoi(argv[1]), streams = std::atoi(argv[2]), percent = std::atoi(argv[3]);
   std::mt19937 rng(seed);
-  nsmi::XcdPlaces<int> places;
+  const unsigned first = rng();
+  nsmi::XcdPlaces<int> places(first);
+  if (nsmi::XcdPlaces<int>(first).one_xcd(1).xcd != int(first % 8)) return std::printf("first XCD\n"), 1;
   Past past[N], queued[64], device_past;     // before launch i; on a stream so far; the last group over the device
   int xcd[N];                                // -1: over the device
   for (int i = 0; i < N; ++i) {
