@@ -127,8 +127,9 @@ int nsmi_pool_trim(nsmi_ctx* ctx);
 /* Failure injection for tests (no counterpart in the reference): the next `count`
    one-launch reductions of this context that run on several workgroups (the
    tridiagonalisation and the bidiagonalisation behind nsmi_factorize) start with
-   their barrier-timeout flag raised, so every workgroup leaves at its first grid
-   barrier and the call reports NSMI_ERR_SOLVER, exactly as when a barrier wait
+   their timeout flag raised: one workgroup leaves before its first column, every
+   other one in its first exchange, when it sees the flag, and the call reports
+   NSMI_ERR_SOLVER with the column, exactly as when a wait for the other workgroups
    gives up; the context stays usable. */
 int nsmi_inject_barrier_timeout(nsmi_ctx* ctx, int count);
 /* The same for their placement: the next `count` of them do not get the XCDs that they ask

@@ -100,6 +100,7 @@ __global__ __launch_bounds__(64 * NW, bidiag_occupancy(NW, MODE)) void k_bidiag(
     G = kXcds * GW;
     g = ww * kXcds + xx;
   }
+  if (MODE != kOneGroup && told_to_give_up(ctl, g)) return;
   constexpr int SP = 64 * CL, SLOTS = ALL ? 32 * kXcds : GMAX;
   double* const PS = xch;                               // [SLOTS][3][SP], an XCD's workgroups together
   double* const Yx = PS + 3 * SLOTS * SP;               // [3][SP]
@@ -387,7 +388,9 @@ __global__ __launch_bounds__(64 * NW, bidiag_occupancy(NW, MODE)) void k_bidiag(
     }
     return true;
   };
-  if (!column_blocks<CL, STEP>(s, s, cb, block)) return;
+  const bool done = column_blocks<CL, STEP>(s, s, cb, block);
+  if (MODE != kOneGroup && tid == 0 && (!done || g == 0)) ended_at(ctl, done ? s : cb);
+  if (!done) return;
   if (lane == 0 && !finite) ctl[kCtlNonFinite] = 1u;
 }
 

@@ -87,7 +87,8 @@ bool one_xcd_groups(nsmi_ctx* ctx) {
   return xcds == kXcds && ncu >= kXcds * XcdPlaces<hipStream_t>::kCusPerXcd;
 }
 
-void reduction_readback(nsmi_ctx* ctx, SytrdRun& run) {
+void reduction_readback(nsmi_ctx* ctx, SytrdRun& run, int columns) {
+  run.columns = columns;
   run.host_flags = static_cast<unsigned*>(stage_take(ctx, kCtlHostWords * sizeof(unsigned)));
   for (int i = 0; i < kCtlHostWords; ++i) run.host_flags[i] = 0u;
   NSMI_HIP(hipMemcpyAsync(run.host_flags, run.flags->as<unsigned>() + kCtlFail, kCtlHostWords * sizeof(unsigned),
@@ -203,7 +204,7 @@ bool bidiag_launch(nsmi_ctx* ctx, double* X, int r, int s, double* d, double* e,
       });
     }
   }
-  reduction_readback(ctx, run);
+  reduction_readback(ctx, run, s);
   return true;
 }
 

@@ -325,13 +325,18 @@ bool sytrd_launch(nsmi_ctx* ctx, double* A, int n, double* d, double* e, double*
       });
     }
   }
-  reduction_readback(ctx, run);
+  reduction_readback(ctx, run, n);
   return true;
 }
 
 void sytrd_check(const SytrdRun& run) {
-  if (run.host_flags[0] || reduction_unplaced(run))
-    fail(NSMI_ERR_SOLVER, "sytrd: a workgroup of the tridiagonal reduction timed out at a grid barrier");
+  if (reduction_unplaced(run))
+    fail(NSMI_ERR_SOLVER, "factorize: the workgroups of the one-launch reduction found no room on the device");
+  // each column's exchange, where every workgroup waits for all the others, is the barrier
+  if (run.host_flags[0])
+    fail(NSMI_ERR_SOLVER, "factorize: a workgroup of the one-launch reduction timed out at a grid barrier (of " +
+                              std::to_string(run.columns) + " columns, in those from " +
+                              std::to_string(run.host_flags[kCtlColumn - kCtlFail]) + " on)");
   // the tridiagonal solver is never handed NaN or Inf
   if (run.host_flags[1]) fail(NSMI_ERR_NOT_FINITE, "factorize: non-finite entries in the matrix to be factorized");
 }

@@ -92,6 +92,13 @@ __device__ __forceinline__ bool load_words(double (&v)[N], const Addr& addr, uns
   }
 }
 
+// the host raised the failure flag before the launch (an injected time-out): the first
+// workgroup of the group leaves at once, and all the others once their polls see the flag
+__device__ inline bool told_to_give_up(const unsigned* ctl, int g) { return g == 0 && ld_agent(ctl + kCtlFail) != 0u; }
+// one lane's record of where the reduction ended (the column itself, kept for this, costs the
+// register-full plans spills)
+__device__ inline void ended_at(unsigned* ctl, int column) { atomicMax(ctl + kCtlColumn, unsigned(column)); }
+
 // ---- placement.  No workgroup of a group does any work before the group's placement is
 // decided, once, by a compare-and-swap of kCtlPlaced from 0: placed when all of the group's
 // workgroups are on the device, unplaced when that cannot be or takes too long; then all of

@@ -428,10 +428,12 @@ void small_sym_eigh(int n, const double* A, double* w, double* V);  // host Jaco
 constexpr int kSytrdMax = 1024;
 //
 // Control words of a reduction (zero on entry): the words the host reads (an exchange that
-// timed out, non-finite d or e, the state of the placement), then the counters of the
-// placement, each on its own 128-byte line (all workgroups, one ticket line per XCD).
+// timed out, non-finite d or e, the state of the placement, the first column of the last block
+// of 64 in which a workgroup gave up, or the number of columns once the first workgroup has
+// finished), then the counters of the placement, each on its own 128-byte line (all
+// workgroups, one ticket line per XCD).
 constexpr int kXcds = 8;
-constexpr int kCtlFail = 32, kCtlNonFinite = 33, kCtlPlaced = 34, kCtlHostWords = 3;
+constexpr int kCtlFail = 32, kCtlNonFinite = 33, kCtlPlaced = 34, kCtlColumn = 35, kCtlHostWords = 4;
 constexpr int kCtlArrived = 64, kCtlTicket = 96;
 constexpr int kCtlWords = kCtlTicket + 32 * kXcds;
 constexpr unsigned kPlaced = 1, kUnplaced = 2;  // kCtlPlaced once it is decided (group.h)
@@ -440,6 +442,7 @@ constexpr unsigned kPlaced = 1, kUnplaced = 2;  // kCtlPlaced once it is decided
 struct SytrdRun {
   std::unique_ptr<Scratch> xch, flags;
   unsigned* host_flags = nullptr;  // in pinned stage memory
+  int columns = 0;
 };
 // spread: the workgroups of a group go wherever there is room and not to one XCD
 bool sytrd_launch(nsmi_ctx* ctx, double* A, int n, double* d, double* e, double* tau, SytrdRun& run,
@@ -456,13 +459,14 @@ bool take_misplacement(nsmi_ctx* ctx);
 // nothing launched, when the device cannot hold all of its grid
 bool launch_over_device(nsmi_ctx* ctx, const void* fn, int groups, int threads, void** args);
 // enqueues the host copy of a launched reduction's control words
-void reduction_readback(nsmi_ctx* ctx, SytrdRun& run);
+void reduction_readback(nsmi_ctx* ctx, SytrdRun& run, int columns);
 // once the copy has arrived: whether the group never started (nothing written; launch again,
 // spread, kRelaunches times)
 constexpr int kRelaunches = 4;
 inline bool reduction_unplaced(const SytrdRun& run) { return run.host_flags[kCtlPlaced - kCtlFail] == kUnplaced; }
 // start value of a reduction's failure flag: 1 when the context has an injected timeout
-// pending and the grid has G > 1
+// pending and the grid has G > 1 (the first workgroup then gives up before its first column,
+// and the others in their first exchange)
 unsigned reduction_fail0(nsmi_ctx* ctx, int G);
 void sytrd_check(const SytrdRun& run);
 // Zr <- (Q Z) with Q = H_0 ... H_{n-2} the reflectors of sytrd_launch's output (rho,

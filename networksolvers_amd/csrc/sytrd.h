@@ -48,7 +48,7 @@ __global__ __launch_bounds__(64 * NW, CL > 8 ? 1 : NW / 2) void k_sytrd(
   unsigned* const fail = ctl + kCtlFail;
   const bool local = want >= 0;  // else a group over all XCDs: the words go past L2
   const int g = local ? place_one_xcd(ctl, G, want, &s_place) : place_spread(ctl, &s_place);
-  if (g < 0) return;
+  if (g < 0 || told_to_give_up(ctl, g)) return;
   double* const P = xch;            // [3][SP]
   double* const Y = xch + 3 * SP;   // [3][SP]
 
@@ -272,6 +272,7 @@ __global__ __launch_bounds__(64 * NW, CL > 8 ? 1 : NW / 2) void k_sytrd(
   };
   const bool done = column_blocks<CL, STEP>(n - 1, n, cb, block);
   if ((done || left) && lane == 0 && !finite) ctl[kCtlNonFinite] = 1u;
+  if (lane == 0 && (g == 0 || !(done || left))) ended_at(ctl, done || left ? n : cb);
 }
 
 }  // namespace

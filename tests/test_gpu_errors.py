@@ -172,7 +172,7 @@ _MANY_SHAPES = [(80, 90), (100, 110), (120, 100), (150, 160), (200, 180), (256, 
 def test_sector_factorize_many_sectors(ctx):
     """Nine sectors spread over the auxiliary streams: every sector's factors equal
     the oracle's (kept counts, U^T U = I, the truncated product U C), a NaN in one
-    sector is reported as NSMI_ERR_NOT_FINITE, a barrier give-up forced from the host
+    sector is reported as NSMI_ERR_NOT_FINITE, a give-up forced from the host
     (the timeout flag of the first multi-workgroup reduction raised before its launch)
     as NSMI_ERR_SOLVER, and after each the same context factorises exactly."""
     from networksolvers_amd import qn
@@ -193,6 +193,7 @@ def test_sector_factorize_many_sectors(ctx):
     with pytest.raises(NsmiError, match="timed out at a grid barrier") as err:
         qn._factorize_sectors(ctx, ctx.upload(buf), offs, rows, cols, False, 1e-10, None, 1, "eigen")
     assert err.value.code == -4
+    assert "columns, in those from 0 on)" in str(err.value)
     _check_sectors(ctx, mats, offs, buf, _MANY_SHAPES)
 
 
@@ -289,13 +290,16 @@ def test_frees_from_other_threads_while_the_owner_computes():
 
 
 @pytest.mark.parametrize("m,n,route", [(100, 110, "eigen"), (300, 320, "eigen"), (200, 220, "svd"),
-                                       (700, 700, "svd"), (1500, 1500, "svd"), (2048, 1024, "svd")])
+                                       (700, 700, "svd"), (1500, 1500, "svd"), (2048, 1024, "svd"),
+                                       (128, 100, "svd"), (512, 512, "svd"), (512, 520, "eigen"), (600, 610, "eigen")])
 def test_reduction_barrier_give_up_is_reported_and_recovered(ctx, m, n, route):
-    """The one-launch reductions wait at grid barriers with a bounded spin; when a
-    wait gives up, every workgroup leaves and the call reports NSMI_ERR_SOLVER.  The
-    host forces that path (the timeout flag is raised before the launch, so each
-    workgroup leaves at its first barrier), then the same context factorises the
-    same matrix correctly."""
+    """In every column of the one-launch reductions each workgroup waits for all the
+    others, with a bounded number of polls; when a wait gives up, every workgroup
+    leaves and the call reports NSMI_ERR_SOLVER.  The host forces that path: the
+    timeout flag is raised before the launch, the first workgroup then leaves before
+    its first column, and the others, waiting for it, in theirs (the error names the
+    last block of columns that any of them got to: the first one).  Then the same
+    context factorises the same matrix correctly."""
     import networksolvers_amd as ns
     from networksolvers_amd._lib import NsmiError
     M = _graded(m, n, 3)
@@ -304,4 +308,5 @@ def test_reduction_barrier_give_up_is_reported_and_recovered(ctx, m, n, route):
     with pytest.raises(NsmiError, match="timed out at a grid barrier") as err:
         ns.factorize(ctx.upload(M.reshape(m, 1, 1, n)), 2, False, cutoff=1e-9, which_decomp=route)
     assert err.value.code == -4
+    assert f"(of {min(m, n)} columns, in those from 0 on)" in str(err.value)
     _factorize_still_works(ctx, m, n, route)
