@@ -491,7 +491,8 @@ bool bidiag_launch(nsmi_ctx* ctx, double* X, int r, int s, double* d, double* e,
 // the Golub-Kahan off-diagonal (d_0, e_0, d_1, ..., d_{s-1}) of the bidiagonal (2 s - 1 entries)
 void gk_offdiag(nsmi_ctx* ctx, const double* d, const double* e, int s, double* gk);
 // eigenvalues of descending rank i0 .. i0 + count - 1 of the symmetric tridiagonal
-// (diagonal a, zero when null; off-diagonal b), N <= kTriSolveMaxN, into lam (device)
+// (diagonal a, zero when null; off-diagonal b), N <= kTriSolveMaxN (with a diagonal N <= 4081),
+// into lam (device)
 constexpr int kTriSolveMaxN = 4096;
 void tri_bisect(nsmi_ctx* ctx, const double* a, const double* b, int N, int i0, int count, double* lam);
 // eigenvectors for the m eigenvalues lam (device) by inverse iteration, as columns of Y

@@ -99,11 +99,18 @@ __device__ __forceinline__ double div_sub(double y, double m, double c) {
   return fma(y * r, fma(e, e, e), fma(y, r, -c));
 }
 
+// steps of a block, and the LDS of `steps` padded steps (16 bytes each)
+constexpr int kB = 8;
+constexpr size_t bisect_lds(int steps) { return 16 * size_t((steps + kB - 1) / kB * kB + kB); }
+// 64 KiB with the kernel's 32 static bytes: order 4081 with a diagonal, 4096 without
+constexpr size_t kBisectLds = 64 * 1024 - 32;
+static_assert(bisect_lds(kSytrdMax - 1) <= kBisectLds && bisect_lds(kTriSolveMaxN / 2) <= kBisectLds,
+              "the tridiagonal reduction's largest order and the Golub-Kahan one's");
+
 template <bool GK>
 __global__ __launch_bounds__(256) void k_tri_bisect(const double* __restrict__ a, const double* __restrict__ b, int N,
                                                     int i0, int count, double* __restrict__ lam) {
   // (d_i^2, e_i^2) of pair i (GK), or (b_i^2, a_{i+1}) of step i, padded to whole blocks
-  constexpr int kB = 8;
   extern __shared__ __align__(16) double sm[];
   double2* const st = reinterpret_cast<double2*>(sm);
   __shared__ double redb[4];
@@ -741,7 +748,8 @@ void tri_bisect(nsmi_ctx* ctx, const double* a, const double* b, int N, int i0, 
   require(a || (N % 2 == 0 && i0 + count <= N / 2), "tridiagonal eigensolver: Golub-Kahan range");
   if (count == 0) return;
   const int steps = a ? N - 1 : N / 2;
-  const size_t shm = sizeof(double) * 2 * size_t((steps + 7) / 8 * 8 + 8);
+  const size_t shm = bisect_lds(steps);
+  require(shm <= kBisectLds, "tridiagonal eigensolver: order above what its LDS holds");
   ProfScope ps(ctx, NSMI_K_FACT_SOLVE, 0.0, 0.0);
   const dim3 grid(unsigned((count + 3) / 4)), block(256);
   if (a)
