@@ -316,7 +316,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_mfma(GemmArgs<T, TBm, TCm> g) 
       for (int r = 0; r < 4; ++r) {
         const int64_t gm = m0 + wm * WTM + i * 16 + out_row<T>(kl, r);
         const int64_t gn = n0 + wn * WTN + j * 16 + ml;
-        if (g.part) {
+        if (BM == 32 && BN == 32 && g.part) {  // only this tile splits K
           if (gm < g.M && gn < g.N) g.part[(int64_t(blockIdx.y) * g.M + gm) * g.N + gn] = acc[i][j][r];
         } else if (gm < g.M && gn < g.N) {
           T v = g.alpha * acc[i][j][r];
@@ -439,24 +439,24 @@ __global__ __launch_bounds__(512) void k_gemm_wave(GemmArgs<T, TBm, TCm> g) {
   C[gm * g.ldc + gn] = TCm(v);
 }
 
-// number of K splits: only for single products whose tile grid leaves most CUs idle
-// and whose K is long; each split keeps at least four K stages
-template <int BM, int BN>
-int splitk_count(const GemmDesc& d, int64_t tiles) {
-  constexpr int BK = (BM == 32 && BN == 32) ? 32 : 16;
+// number of K splits of the 32 x 32 tile: only for single products whose tile grid leaves most
+// CUs idle and whose K is long; each split keeps at least four K stages.  (The larger tiles
+// are taken from 205 and 448 of them on, where there is nothing to split.)
+constexpr int kSplitBk = 32;
+inline int splitk_count(const GemmDesc& d, int64_t tiles) {
   if (d.batch != 1 || tiles >= 128) return 1;
-  const int64_t stages = (d.K + BK - 1) / BK;
+  const int64_t stages = (d.K + kSplitBk - 1) / kSplitBk;
   const int64_t by_grid = 512 / tiles, by_k = stages / 4;
   return int(std::max<int64_t>(1, std::min<int64_t>({by_grid, by_k, int64_t(8)})));
 }
 
 template <typename T, typename TBm, typename TCm, int BM, int BN, int ROLE>
 void launch_tile(nsmi_ctx* ctx, const GemmDesc& d, GemmArgs<T, TBm, TCm>& a) {
-  constexpr int BK = (BM == 32 && BN == 32) ? 32 : 16;
+  constexpr bool kSplit = BM == 32 && BN == 32;
   a.tiles_m = int((d.M + BM - 1) / BM);
   a.tiles_n = int((d.N + BN - 1) / BN);
-  const int S = splitk_count<BM, BN>(d, int64_t(a.tiles_m) * a.tiles_n);
-  a.kc = S == 1 ? std::max<int64_t>(d.K, 1) : ((d.K + S - 1) / S + BK - 1) / BK * BK;
+  const int S = kSplit ? splitk_count(d, int64_t(a.tiles_m) * a.tiles_n) : 1;
+  a.kc = S == 1 ? std::max<int64_t>(d.K, 1) : ((d.K + S - 1) / S + kSplitBk - 1) / kSplitBk * kSplitBk;
   const int splits = int((d.K + a.kc - 1) / a.kc);
   std::unique_ptr<Scratch> part;
   a.part = nullptr;
