@@ -529,7 +529,7 @@ void fact_emit(nsmi_ctx* ctx, FactCore& f, int64_t k, double* U, double* C) {
                   f.want_v ? 0 : 1);
       else
         tri_invit(ctx, f.w->as<double>(), f.e->as<double>(), int(iso), lamk.as<double>(), int(k), Y.as<double>(), -1);
-      unsigned* ofail = f.sr.flags->as<unsigned>() + 40;
+      unsigned* ofail = f.sr.flags->as<unsigned>() + kCtlOrthFail;
       orthonormalize_cols(ctx, Y.as<double>(), len, int(k), ofail);
       f.orth_h = static_cast<unsigned*>(stage_take(ctx, sizeof(unsigned)));
       *f.orth_h = 0u;

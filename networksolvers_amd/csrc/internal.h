@@ -430,10 +430,12 @@ constexpr int kSytrdMax = 1024;
 // Control words of a reduction (zero on entry): the words the host reads (an exchange that
 // timed out, non-finite d or e, the state of the placement, the first column of the last block
 // of 64 in which a workgroup gave up, or the number of columns once the first workgroup has
-// finished), then the counters of the placement, each on its own 128-byte line (all
-// workgroups, one ticket line per XCD).
+// finished), then the flag of the orthonormalisation that follows in the same call
+// (orthonormalize_cols), then the counters of the placement, each on its own 128-byte line
+// (all workgroups, one ticket line per XCD).
 constexpr int kXcds = 8;
 constexpr int kCtlFail = 32, kCtlNonFinite = 33, kCtlPlaced = 34, kCtlColumn = 35, kCtlHostWords = 4;
+constexpr int kCtlOrthFail = 40;
 constexpr int kCtlArrived = 64, kCtlTicket = 96;
 constexpr int kCtlWords = kCtlTicket + 32 * kXcds;
 constexpr unsigned kPlaced = 1, kUnplaced = 2;  // kCtlPlaced once it is decided (group.h)
