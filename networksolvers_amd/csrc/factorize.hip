@@ -335,6 +335,7 @@ void fact_tri_solve(nsmi_ctx* ctx, FactCore& f) {
     NSMI_HIP(hipStreamSynchronize(ctx->stream));
   }
   sytrd_check(f.sr);
+  f.sr.xch.reset();
   f.lam.reset(new Scratch(ctx, sizeof(double) * size_t(iso)));
   tri_bisect(ctx, f.w->as<double>(), f.e->as<double>(), int(iso), 0, int(iso), f.lam->as<double>());
   f.wh = static_cast<double*>(stage_take(ctx, sizeof(double) * size_t(iso)));
@@ -482,6 +483,7 @@ void fact_prepare(nsmi_ctx* ctx, FactCore& f) {
       if (launched) NSMI_HIP(hipStreamSynchronize(ctx->stream));
     }
     if (launched) {
+      f.sr.xch.reset();  // up to 13 MB over all XCDs; the vectors' solves that follow need the most
       fact_finish(f);
       return;
     }

@@ -162,6 +162,22 @@ def test_misplaced_sector_groups_give_the_same_result(ctx):
     np.testing.assert_array_equal(c, c1)
 
 
+@pytest.mark.parametrize("m,n,route,limit", [(250, 250, "svd", 4506624), (422, 394, "svd", 15894016),
+                                             (600, 600, "svd", 32049664), (1000, 800, "svd", 61934080),
+                                             (2048, 2048, "svd", 312611328), (700, 710, "eigen", 27339264)])
+def test_factorisation_fits_the_pool_it_fitted(m, n, route, limit):
+    """Pool limits that held a factorisation with k = n / 2 when the reductions' exchange was
+    smaller (two buffers, 8 to 256 workgroups) still hold it: the exchange is given back before
+    the vectors' solves, where the peak is."""
+    import networksolvers_amd as ns
+    c = ns.Context(0)
+    x = c.upload(np.random.default_rng(1).standard_normal((m, n)))
+    ns.factorize(x, 1, False, cutoff=0.0, maxdim=min(m, n) // 2, which_decomp=route)
+    assert c.pool_stats()["peak"] <= limit
+    del x
+    c.close()
+
+
 def _same_from_threads(ctx, ctxs, work, rounds):
     """Every context factorises the matrices of `work` in turn, five threads sharing the
     contexts; C is compared with that of `ctx` alone."""
