@@ -31,7 +31,7 @@ HBM_PEAK_GBS = 8000.0
 # launches themselves, on the context stream): the roofline is reported for the one
 # with the largest summed time.  name -> (kernel, bound, unit of the peak)
 ROOF_CLASSES = {
-    "fact_reduce": "k_bidiag / k_sytrd_* (one-launch bidiagonalisation / tridiagonalisation of factorize)",
+    "fact_reduce": "k_bidiag / k_sytrd (one-launch bidiagonalisation / tridiagonalisation of factorize)",
     "heff_gemm1": "k_gemm_mfma H_eff GEMM1 (L . theta)",
     "heff_gemm2": "k_gemm_mfma H_eff GEMM2 (T3 . R^T, split-K reduction included)",
 }
