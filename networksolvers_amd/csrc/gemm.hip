@@ -190,8 +190,8 @@ template <typename T, typename TBm, typename TCm, int BM, int BN, bool TA, bool 
 __global__ __launch_bounds__(64 * NW) void k_gemm_mfma(GemmArgs<T, TBm, TCm> g) {
   // the small tiles run twice as deep a K slice per LDS stage: the products they
   // serve have few tiles and long K, so the per-stage barrier and load latency is
-  // what they pay (measured on the FP32 H_eff GEMM2 at 852 x 213 x 1065: 38.8 us
-  // at depth 16, 27.7 us at 32, 30.8 us at 64)
+  // what they pay (measured on the FP32 H_eff GEMM2 at 852 x 213 x 1065 with loads one
+  // slab ahead: 38.8 us at depth 16, 27.7 us at 32, 30.8 us at 64)
   constexpr int BK = (BM == 32 && BN == 32) ? 32 : 16;
   constexpr int NT = 64 * NW, GM = 2, GN = NW / 2;
   constexpr int WTM = BM / GM, WTN = BN / GN;

@@ -1,4 +1,4 @@
-// Exchange between the workgroups of the one-launch reductions (bidiag.h, eig.hip).
+// Exchange between the workgroups of the one-launch reductions (bidiag.h, sytrd.h).
 //
 // A grid barrier with an agent-scope release and acquire writes back and invalidates
 // L2 lines; measured (256 threads per workgroup, in-bounds probe): 1.0 us at 12
@@ -67,11 +67,12 @@ __device__ inline void st_group(double* p, double v, bool local) {
 // this wave's stores have reached the level their readers load from
 __device__ inline void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// Loads N words, addr(i) their addresses, until none is empty.  The first round loads all
-// of them at once; later rounds only what is still missing: rounds that reload
-// everything keep the L2 so busy that the awaited stores take 10x longer (394 columns,
-// 14 workgroups of one XCD: 36 us per step against 3).  False once it gives up (the
-// failure flag raised) or another workgroup has raised the flag.
+// Loads N words, addr(i) their addresses, until none is empty: all of them again in every
+// round, with a pause of 256 cycles between rounds.  Without the pause the polls keep the L2
+// so busy that the awaited stores take 10x longer (394 columns, 14 workgroups of one
+// XCD: 36 us per step against 3); loading only what is still missing needs branches and took
+// 5.5.  False once it gives up (the failure flag raised) or another workgroup has raised the
+// flag.
 template <int N, class Addr>
 __device__ __forceinline__ bool load_words(double (&v)[N], const Addr& addr, unsigned* fail) {
   for (unsigned spins = 0;;) {
@@ -110,7 +111,7 @@ __device__ inline void decide(unsigned* ctl, unsigned state) {
                                        __HIP_MEMORY_SCOPE_AGENT);
   stores_done();
 }
-// one lane's wait for the decision, about half a second at most
+// one lane's wait for the decision: a million polls (tenths of a second) at most
 __device__ inline bool placed(unsigned* ctl) {
   for (unsigned spins = 0;; ++spins) {
     const unsigned state = ld_agent(ctl + kCtlPlaced);
@@ -204,8 +205,9 @@ __global__ void k_reduction_init(double* __restrict__ xch, size_t n, size_t ps, 
 // A Householder reflector's scalars for [alpha, x] with sigma2 = |x|^2 (LAPACK dlarfg):
 // beta = -sign(alpha) sqrt(alpha^2 + sigma2), tau = (beta - alpha) / beta, scal = 1 /
 // (alpha - beta).  With n = sqrt(alpha^2 + sigma2): tau = (n + |alpha|) / n, scal =
-// sign(alpha) / (n + |alpha|), no cancellation.  1 / n by the hardware reciprocal
-// square root and two coupled Newton steps, n corrected by its residual, 1 / (n +
+// sign(alpha) / (n + |alpha|), no cancellation.  1 / n and n by Goldschmidt's iteration
+// from the hardware reciprocal square root (g -> n and h -> 1 / (2 n) take the same factor
+// 1 + e, e = 1/2 - g h, twice), n corrected by its residual, 1 / (n +
 // |alpha|) by the refined reciprocal: each within an ulp or two, on a dependency chain
 // less than half as long as a rounded square root and two divisions (450 cycles).
 __device__ inline void reflector(double alpha, double sigma2, double* beta, double* tau, double* scal) {

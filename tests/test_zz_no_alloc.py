@@ -6,8 +6,9 @@ split, so its result must equal the allocating apply bit for bit.  Two calls in 
 row on the shared array, the second with a smaller operator (the array keeps the
 first call's contents), in the FP64 and FP32 forms, at shapes whose GEMM2 is split
 over K (chi = 150: 600 x 150 output on 95 tiles of 32 x 32, K = 750 in 5 splits;
-chi 90 x 70: 36 tiles, K = 350 in 2 splits); an operator form it does not serve is
-rejected.
+chi 130 x 120: 520 x 120 on 68 tiles, K = 600 in 4), then one whose products need no
+partial sums in memory (chi 90 x 70: 36 tiles, K = 350, the one-block form); an operator
+form it does not serve is rejected.
 """
 import ctypes as C
 
@@ -36,7 +37,7 @@ def test_noalloc_apply_equals_apply(precision, bar):
     ctx = ns.Context(0)
     try:
         assert ctx.lib.nsmi_noalloc_scratch_bytes() == 32 << 20
-        for cl, cr, seed in [(150, 150, 1), (90, 70, 2)]:
+        for cl, cr, seed in [(150, 150, 1), (130, 120, 3), (90, 70, 2)]:
             print(f"noalloc apply {precision} chi_l={cl} chi_r={cr}", flush=True)
             H, x, want = _case(ctx, cl, cr, precision, seed)
             y_ref = H(x).numpy()
