@@ -3,6 +3,7 @@
 // kernel is k_sytrd (sytrd.h), its plans and launch below; the batched Jacobi solver for
 // small Gram matrices; and the compact-WY back-transformation of the kept vectors.
 #include "internal.h"
+#include "places.h"
 #include "sytrd.h"
 #include "wave.h"
 
@@ -14,9 +15,12 @@ struct TriPlan {
   int cl = 1, threads = 0, rows = 0;  // rows per workgroup
   bool spread = false;                // over all XCDs
 };
-template <int CL, int RW, int NW, bool SHARED>
-TriPlan tri_plan_of(bool spread = false) {
-  return {reinterpret_cast<const void*>(k_sytrd<CL, RW, NW, SHARED>), CL, 64 * NW, RW * NW, spread};
+template <int NMAX, int CL, int RW, int NW, bool SHARED>
+TriPlan tri_plan_of() {
+  constexpr bool kSpread = CL > 8;  // as the kernel's register bound
+  static_assert(NMAX <= 64 * CL && (kSpread || NMAX <= XcdPlaces<hipStream_t>::kCusPerXcd * RW * NW),
+                "at most one workgroup for each CU of an XCD");
+  return {reinterpret_cast<const void*>(k_sytrd<CL, RW, NW, SHARED>), CL, 64 * NW, RW * NW, kSpread};
 }
 
 // Measured on gfx950 (us per column; the grid-barrier form on up to 16 spread workgroups
@@ -28,11 +32,11 @@ TriPlan tri_plan_of(bool spread = false) {
 // spills (4.8 at 700, 9 at 1000), so the group spreads over all XCDs: 3.3 at 513, 3.7 at
 // 700, 4.3 at 1000.
 TriPlan tri_plan(int n) {
-  if (n <= 64) return tri_plan_of<1, 1, 4, false>();
-  if (n <= 128) return tri_plan_of<2, 1, 4, false>();
-  if (n <= 256) return tri_plan_of<4, 2, 4, false>();
-  if (n <= 512) return tri_plan_of<8, 4, 4, false>();
-  return tri_plan_of<16, 2, 4, true>(true);
+  if (n <= 64) return tri_plan_of<64, 1, 1, 4, false>();
+  if (n <= 128) return tri_plan_of<128, 2, 1, 4, false>();
+  if (n <= 256) return tri_plan_of<256, 4, 2, 4, false>();
+  if (n <= 512) return tri_plan_of<512, 8, 4, 4, false>();
+  return tri_plan_of<kSytrdMax, 16, 2, 4, true>();
 }
 
 // ---- batched Jacobi eigensolver for small Gram matrices ---------------------
