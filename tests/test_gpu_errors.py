@@ -163,8 +163,8 @@ def _check_sectors(ctx, mats, offs, buf, shapes):
         co += k * n
 
 
-# sectors on every reduction plan of the Gram sizes 65..320 (three each on the 65..128
-# and 129..256 plans), one on the one-workgroup plan (60), one Jacobi (30)
+# sectors on every one-XCD reduction plan (three each on the 65..128 and 129..256 plans, one
+# above, one on the 41..64 plan), one Jacobi (30)
 _MANY_SHAPES = [(80, 90), (100, 110), (120, 100), (150, 160), (200, 180), (256, 256), (300, 320), (60, 70),
                 (30, 35)]
 

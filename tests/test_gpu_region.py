@@ -243,9 +243,9 @@ def test_factorize(ctx, route, trailing, shape, cutoff, maxdim):
 def test_factorize_eigensolver_paths(ctx, m, n, maxdim):
     """Gram sizes across every eigensolver path, with a graded spectrum: the
     batched Jacobi solver for small Gram matrices, every plan of the one-launch
-    tridiagonal reduction (one workgroup to 64; 4, 4, 6, 7, 8 rows per wave to 128,
-    256, 384, 448, 512 on up to 16 workgroups; the cooperative grid to 1024) on both
-    sides of each boundary, and rocSOLVER dsyevd above 1024."""
+    tridiagonal reduction (1, 1, 2, 4 rows per wave to 64, 128, 256, 512 on up to 32
+    workgroups of one XCD; two rows per wave over all XCDs to 1024) on both sides of
+    each boundary, and rocSOLVER dsyevd above 1024."""
     import networksolvers_amd as ns
     rng = np.random.default_rng(m + n)
     r = min(m, n)
@@ -358,16 +358,15 @@ def _graded_matrix(m, n, decay, seed, degenerate=1):
                                  (2500, 400), (2048, 1024), (4096, 600)])
 def test_svd_route_bidiagonal_paths(ctx, m, n):
     """The svd route (bidiagonalisation + Golub-Kahan bisection + inverse iteration)
-    on every plan of the one-launch bidiagonalisation (one workgroup to 64 x 64; 1, 2,
-    4, 8, 16, 32 columns per lane; plain and cooperative grids), tall and wide: the
+    over the range of the one-launch bidiagonalisation (one workgroup, one XCD, all
+    XCDs; 1, 2, 4, 8, 16, 32 columns per lane), tall and wide: the
     spectrum P = s^2 of an SVD to 1e-13 of P_max, U^T U = I, U C = the oracle's
     (numpy SVD) truncated product, singular vectors element-wise where resolved, and
-    the route that ran is the svd route (no Gram fallback).  Grids of up to 64
-    workgroups exchange in one level; the two-level exchange runs at 188 and 256
-    workgroups with 32 columns per lane (1100 x 1500, 2048 x 2048), at 79 with 8
-    (2500 x 400) and at 128 and 256 with 16 (2048 x 1024, the chain's 1024 | 512 bond
-    regions, and 4096 x 600); the inverse iteration keeps its factors in global memory
-    from Golub-Kahan order 1025 on."""
+    the route that ran is the svd route (no Gram fallback).  Groups over all XCDs run
+    with 24 and 32 workgroups on each for 32 columns per lane (1500 x 1100, 2048 x
+    2048), with 20 for 8 (2500 x 400) and with 32 for 16 (2048 x 1024, the chain's 1024 |
+    512 bond regions, and 4096 x 600); the inverse iteration keeps its factors in global
+    memory from Golub-Kahan order 1025 on."""
     import networksolvers_amd as ns
     M = _graded_matrix(m, n, 8.0, m * 7 + n)
     maxdim = max(1, min(m, n) // 2)
