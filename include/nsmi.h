@@ -134,8 +134,9 @@ int nsmi_pool_trim(nsmi_ctx* ctx);
 int nsmi_inject_barrier_timeout(nsmi_ctx* ctx, int count);
 /* The same for their placement: the next `count` of them do not get the XCDs that they ask
    for.  A group on one XCD then leaves without having started and is launched again over
-   the whole device; a group over all XCDs is formed in the grid's order.  Results are
-   those of the usual placement, bit for bit. */
+   the whole device (with count 2 that placement times out, and it is launched once more);
+   a group over all XCDs is formed in the grid's order.  Results are those of the usual
+   placement, bit for bit. */
 int nsmi_inject_misplacement(nsmi_ctx* ctx, int count);
 
 /* ---------------------------------------------------------------- tensors */

@@ -184,7 +184,7 @@ bool bidiag_launch(nsmi_ctx* ctx, double* X, int r, int s, double* d, double* e,
   const unsigned nblk = unsigned(std::min<size_t>(1024, (std::max<size_t>(x.words, kCtlWords) + 255) / 256));
   hipLaunchKernelGGL(k_reduction_init, dim3(nblk), dim3(256), 0, ctx->stream, xp, x.words, x.ps_words,
                      unsigned(3 * 64 * p.cl), unsigned(std::max(x.per, 1)), unsigned(x.used), ctl, int(kCtlWords),
-                     reduction_fail0(ctx, G));
+                     reduction_fail0(ctx, G), spread && take_misplacement(ctx) ? kNeverArrived : 0u);
   NSMI_LAUNCH_CHECK();
   int rr = r, ss = s, want = -1;
   void* args[] = {&X, &rr, &ss, &d, &e, &tauL, &tauR, &xp, &ctl, &groups, &want};

@@ -314,7 +314,8 @@ bool sytrd_launch(nsmi_ctx* ctx, double* A, int n, double* d, double* e, double*
   unsigned* ctl = run.flags->as<unsigned>();
   double* xp = run.xch->as<double>();
   hipLaunchKernelGGL(k_reduction_init, dim3(unsigned((std::max<size_t>(words, kCtlWords) + 255) / 256)), dim3(256), 0,
-                     ctx->stream, xp, words, size_t(0), 1u, 1u, 1u, ctl, int(kCtlWords), reduction_fail0(ctx, G));
+                     ctx->stream, xp, words, size_t(0), 1u, 1u, 1u, ctl, int(kCtlWords), reduction_fail0(ctx, G),
+                     spread && take_misplacement(ctx) ? kNeverArrived : 0u);
   NSMI_LAUNCH_CHECK();
   int nn = n, want = -1;
   void* args[] = {&A, &nn, &d, &e, &tau, &xp, &ctl, &G, &want};

@@ -111,7 +111,7 @@ __device__ inline void decide(unsigned* ctl, unsigned state) {
                                        __HIP_MEMORY_SCOPE_AGENT);
   stores_done();
 }
-// one lane's wait for the decision: a million polls (tenths of a second) at most
+// one lane's wait for the decision: a million polls (about a tenth of a second) at most
 __device__ inline bool placed(unsigned* ctl) {
   for (unsigned spins = 0;; ++spins) {
     const unsigned state = ld_agent(ctl + kCtlPlaced);
@@ -191,13 +191,14 @@ __device__ __forceinline__ bool column_blocks(int stop, int width, int& cb, cons
   return true;
 }
 
-// empties the exchange words and zeroes the control words (fail0: the failure flag's
-// start value) before a reduction; the first ps words are slots of `slot` words, of
+// empties the exchange words and zeroes the control words (fail0, arrived0: start values of
+// the failure flag and of the arrival count) before a reduction; the first ps words are slots of `slot` words, of
 // which every group of `per` fills the first `used`: the others become zeros
 __global__ void k_reduction_init(double* __restrict__ xch, size_t n, size_t ps, unsigned slot, unsigned per,
-                                 unsigned used, unsigned* __restrict__ ctl, int nctl, unsigned fail0) {
+                                 unsigned used, unsigned* __restrict__ ctl, int nctl, unsigned fail0,
+                                 unsigned arrived0) {
   const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < size_t(nctl)) ctl[i] = int(i) == kCtlFail ? fail0 : 0u;
+  if (i < size_t(nctl)) ctl[i] = int(i) == kCtlFail ? fail0 : int(i) == kCtlArrived ? arrived0 : 0u;
   for (size_t k = i; k < n; k += size_t(gridDim.x) * blockDim.x)
     xch[k] = k < ps && unsigned(k) / slot % per >= used ? 0.0 : empty_word();
 }

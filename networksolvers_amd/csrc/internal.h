@@ -455,8 +455,10 @@ bool one_xcd_groups(nsmi_ctx* ctx);
 // runs on one XCD: the stream's place among the XCDs, see places.h
 void launch_on_one_xcd(nsmi_ctx* ctx, const std::function<void(int)>& launch);
 void xcd_places_release(int device, hipStream_t stream);
-// whether a placement is to fail, by injection (tests); counts it
+// whether a placement is to fail, by injection (tests); counts it.  A one-XCD group then asks
+// for an XCD that is not there, one launched again starts with an arrival count out of reach
 bool take_misplacement(nsmi_ctx* ctx);
+constexpr unsigned kNeverArrived = 1u << 31;
 // cooperative launch of a group over the device, alone among the groups (places.h); false, with
 // nothing launched, when the device cannot hold all of its grid
 bool launch_over_device(nsmi_ctx* ctx, const void* fn, int groups, int threads, void** args);
